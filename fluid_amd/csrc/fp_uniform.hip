@@ -24,6 +24,7 @@
 #include "fp_sweep.hpp"
 #include "fp_sweep2.hpp"
 #include "fp_march.hpp"
+#include "fp_leg.hpp"
 #include "fp_state.hpp"
 
 #include <algorithm>
@@ -1774,6 +1775,24 @@ void UniformGrid::set_tuning(int tile_z, int groups, int pairs) {
   }
 }
 
+// A level runs as legs (fp_leg.hpp) when its cells over all grids of the
+// launch are at most this many: beyond it the ring's redundant work costs more
+// than the launches that a leg saves, sooner with 4-byte storage (two tiles'
+// LDS do not fit a CU then).  The bits are the same either way, so the choice
+// may depend on what a grid is batched with.  Whole projections, legs against
+// launches on the finest level: FP16 32^3 1.06 / 1.45 ms, 64^3 1.36 / 1.49,
+// 96^3 (0.88 M cells) 1.59 / 1.69, 128^3 (2.1 M) 3.04 / 2.26; FP32
+// 121 x 75 x 98 (0.89 M) 2.26 / 2.13.
+static long long leg_cells(int precision) { return precision == FP_PRECISION_FP32 ? 1ll << 19 : 1ll << 20; }
+
+static int leg_groups(const int* d) {
+  return ((d[0] + kLegX - 1) / kLegX) * ((d[1] + kLegY - 1) / kLegY) * ((d[2] + kLegZ - 1) / kLegZ);
+}
+
+// A projection whose options ask for the finest level's launches one by one:
+// persistent sweeps, or one kernel class timed.
+static bool split_launches(const fp_options* o) { return o->persistent != 0 || o->timed_kernel != FP_KERNEL_NONE; }
+
 void UniformGrid::set_level_scales(int precision, int pre, int post) {
   // FP32: every scale is 1.  FP16/BF16: the finest right-hand side arrives
   // normalised to |r| <= 1 (device rscale); error vectors grow like
@@ -1828,6 +1847,8 @@ struct Projector::Plan {
   long long bottom_n[kMaxLevels] = {};  // per bottom level (from lb): most cells over coarse_deep's grids
   struct Level {
     PartTable sweep32, sweep16;  // fused grids by sweep tile width
+    PartTable leg;               // grids whose level runs as legs; in none of the V-cycle's tables below
+    PartTable hull;              // fused grids: march tiles (set-up)
     PartTable res;               // fused grids: residual march
     PartTable fusedcells;        // fused grids: cells of the level
     PartTable smooth;            // unfused grids: cells of the level
@@ -1897,7 +1918,8 @@ void Projector::forget(int grid_id) {
 }
 
 // Host part tables of a grid set (dev pointers are set by the upload).
-void Projector::fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int precision, int pre, int post) {
+void Projector::fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int precision, int pre, int post,
+                            bool split) {
   p->grids = grids;
   p->precision = precision;
   p->pre = pre;
@@ -1935,18 +1957,37 @@ void Projector::fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int
   p->add(p->coarse_top, ctop);
   p->add(p->coarse_deep, cdeep);
   for (int l = 0; l < maxL; ++l) {
-    Items s32, s16, res, fc, sm, rs, dn;
+    Items s32, s16, leg, hull, res, fc, sm, rs, dn;
+    // the whole level runs as legs or none of it: a leg beside sweeps of the
+    // same level would be one launch more
+    long long fused_cells = 0;
+    bool legs = !split && pre >= 1 && pre <= kLegSweeps && post >= 1 && post <= kLegSweeps;
+    for (UniformGrid* g : grids) {
+      const GridRec& R = *g->host_rec();
+      if (l < R.L - 1 && R.lv[l].fused) {
+        fused_cells += R.lv[l].n;
+        legs = legs && g->sweep_pairs() != 1;
+      }
+    }
+    legs = legs && fused_cells <= leg_cells(precision);
     for (UniformGrid* g : grids) {
       const GridRec& R = *g->host_rec();
       if (l >= R.L) continue;
       const LevelRec& lv = R.lv[l];
       if (l >= 1) dn.push_back({g, Plan::blocks_for((size_t)lv.n, 1)});
       if (l >= R.L - 1) continue;  // the coarsest level is solved directly
+      if (lv.fused) {
+        hull.push_back({g, lv.mg.ngroups});
+        fc.push_back({g, Plan::blocks_for((size_t)lv.n, 1)});
+      }
+      if (legs && lv.fused) {
+        leg.push_back({g, leg_groups(lv.d)});
+        continue;
+      }
       if (l < R.lb) rs.push_back({g, R.lv[l + 1].rg.ngroups});
       if (lv.fused) {
         (lv.sweep_tz == 32 ? s32 : s16).push_back({g, lv.sw.ngroups});
         res.push_back({g, lv.mg.ngroups});
-        fc.push_back({g, Plan::blocks_for((size_t)lv.n, 1)});
       } else if (l < R.lb) {
         sm.push_back({g, Plan::blocks_for((size_t)lv.n, 1)});
       }
@@ -1954,6 +1995,8 @@ void Projector::fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int
     Plan::Level& T = p->lv[l];
     p->add(T.sweep32, s32);
     p->add(T.sweep16, s16);
+    p->add(T.leg, leg);
+    p->add(T.hull, hull);
     p->add(T.res, res);
     p->add(T.fusedcells, fc);
     p->add(T.smooth, sm);
@@ -1974,11 +2017,11 @@ Projector::Plan* Projector::plan_for(const std::vector<UniformGrid*>& grids, con
   key.push_back(opt->precision);
   key.push_back(opt->pre_sweeps);
   key.push_back(opt->post_sweeps);
-  key.push_back(opt->persistent ? 1 : 0);
+  key.push_back((opt->persistent ? 1 : 0) | (split_launches(opt) ? 2 : 0));
   auto it = plans_.find(key);
   if (it != plans_.end()) return it->second;
   Plan* p = new Plan();
-  fill_tables(p, grids, opt->precision, opt->pre_sweeps, opt->post_sweeps);
+  fill_tables(p, grids, opt->precision, opt->pre_sweeps, opt->post_sweeps, split_launches(opt));
   p->persistent = opt->persistent != 0;
   bool ok = hipMalloc((void**)&p->arena, std::max<size_t>(1, p->host.size()) * sizeof(Part)) == hipSuccess;
   ok = ok && hipMemcpy(p->arena, p->host.data(), p->host.size() * sizeof(Part), hipMemcpyHostToDevice) == hipSuccess;
@@ -2077,12 +2120,21 @@ static void sweep2_launch(hipStream_t s, const PartTable& t32, const PartTable& 
   }
 }
 
+#define LEG_LAUNCH(kern, tab, stream, ...)                                                                       \
+  do {                                                                                                           \
+    if ((tab).n > 0)                                                                                             \
+      hipLaunchKernelGGL(kern, dim3((tab).blocks), dim3(kLegThreads), 0, stream, (tab).dev, (tab).n, ##__VA_ARGS__); \
+  } while (0)
+
 template <typename T>
 int Projector::vcycle_t(hipStream_t s, Plan& p) {
   const int pre = p.pre, post = p.post;
   for (int l = 0; l + 1 < p.maxL; ++l) {
     Plan::Level& T_ = p.lv[l];
     const bool top = l == 0;
+    // ---- legs: pre-smoothing, residual and restriction in one launch ----
+    if (top) LEG_LAUNCH((k_leg_down<float, T>), T_.leg, s, l, pre);
+    else LEG_LAUNCH((k_leg_down<T, T>), T_.leg, s, l, pre);
     // ---- pre-smoothing ----
     if (pre == 0) {
       PLAUNCH(k_zero_level<T>, T_.fusedcells, s, l);
@@ -2147,6 +2199,9 @@ int Projector::vcycle_t(hipStream_t s, Plan& p) {
   for (int l = p.maxL - 2; l >= 0; --l) {
     Plan::Level& T_ = p.lv[l];
     const bool top = l == 0;
+    // ---- legs: prolongation and post-smoothing in one launch ----
+    if (top) LEG_LAUNCH((k_leg_up<float, T>), T_.leg, s, l, post);
+    else LEG_LAUNCH((k_leg_up<T, T>), T_.leg, s, l, post);
     // ---- fused levels: prolongation over the liquid hulls, then the sweeps ----
     if (post == 0) {
       PLAUNCH(k_prolong_add<T>, T_.fusedcells, s, l, pre & 1);
@@ -2261,7 +2316,7 @@ int Projector::setup_tables(hipStream_t s, Plan& p, int preserve) {
   else build_weights_t<float>(s, this, p.maxL, wt);
   for (int l = 0; l + 1 < p.maxL; ++l) {
     PLAUNCH(k_hull_reset, p.lv[l].fusedcells, s, l);
-    PLAUNCH(k_tile_hull, p.lv[l].res, s, l);
+    PLAUNCH(k_tile_hull, p.lv[l].hull, s, l);
   }
   return FP_OK;
 }
@@ -2474,7 +2529,8 @@ int Projector::run_noalloc(hipStream_t s, int device, UniformGrid* g, const fp_o
   // the counters
   Plan& p = *noalloc_plan_;
   const std::vector<UniformGrid*> one_grid(1, g);
-  fill_tables(&p, one_grid, opt->precision, opt->pre_sweeps, opt->post_sweeps);
+  // (the entry point never times a kernel class)
+  fill_tables(&p, one_grid, opt->precision, opt->pre_sweeps, opt->post_sweeps, opt->persistent != 0);
   p.persistent = opt->persistent != 0;
   const size_t parts_bytes = p.host.size() * sizeof(Part);
   const size_t state_off = (parts_bytes + 255) & ~(size_t)255;
@@ -2548,7 +2604,7 @@ int Projector::serve_round(hipStream_t s, std::vector<Job*>& jobs) {
     std::vector<UniformGrid*> gs;
     for (Job* j : js) gs.push_back(j->grid);
     plans.emplace_back(new Plan());
-    fill_tables(plans.back().get(), gs, o.precision, o.pre_sweeps, o.post_sweeps);
+    fill_tables(plans.back().get(), gs, o.precision, o.pre_sweeps, o.post_sweeps, o.persistent != 0);
     plans.back()->persistent = o.persistent != 0;
     return plans.back().get();
   };

@@ -299,7 +299,7 @@ class Projector {
   // or the gradient subtract); each stage group is one batched launch set.
   // Jobs whose stage became DONE carry their report.
   int serve_round(hipStream_t s, std::vector<Job*>& jobs);
-  void fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int precision, int pre, int post);
+  void fill_tables(Plan* p, const std::vector<UniformGrid*>& grids, int precision, int pre, int post, bool split);
 
  private:
   Plan* plan_for(const std::vector<UniformGrid*>& grids, const fp_options* opt);

@@ -33,3 +33,20 @@ def test_bottom_matches_oracle(fpl, oracle, dims):
             assert np.linalg.norm(z - oz) < 2e-5 * np.linalg.norm(oz), sweeps
     finally:
         g.destroy()
+
+
+# one tile, ragged tiles, axes that do not coarsen, an odd row length, and both sides of the size limit of FP32 legs
+@pytest.mark.parametrize("dims", [(16, 16, 16), (4, 16, 64), (17, 19, 23), (33, 20, 18), (40, 24, 17), (5, 33, 32),
+                                  (64, 10, 21), (80, 81, 80), (81, 81, 81)])
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
+def test_leg_bits(fpl, dims, precision):
+    phi, r, h = blob_case(dims, sum(dims))
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        for sweeps in (1, 2, 3):
+            z = [g.probe_vcycle(phi, r, precision=precision, pre_sweeps=sweeps, post_sweeps=sweeps, persistent=p)
+                 for p in (0, 1)]
+            assert np.isfinite(z[0]).all() and np.abs(z[0]).max() > 0
+            assert np.array_equal(z[0], z[1]), (sweeps, np.abs(z[0] - z[1]).max())
+    finally:
+        g.destroy()

@@ -1132,6 +1132,8 @@ void TallGrid::release() {
   allocations_.clear();
   if (rec_) (void)hipHostFree(rec_);
   rec_ = nullptr;
+  if (rm_host_) (void)hipHostFree(rm_host_);
+  rm_host_ = nullptr;
 }
 
 int TallGrid::alloc(void** p, size_t bytes) {

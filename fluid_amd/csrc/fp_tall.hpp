@@ -116,7 +116,7 @@ class TallGrid {
   int remesh(hipStream_t s, const fp_tall_remesh_args* a, int64_t* changed_columns);
   // Device bytes the first remesh adds (its staging buffers).
   static size_t remesh_bytes(int nx, int nz, int band, int max_delta);
-  bool remesh_ready() const { return rm_in_ != nullptr; }
+  bool remesh_ready() const { return rm_host_ != nullptr; }
   int levels() const { return rec_->L; }
   const TallLevel& level(int l) const { return rec_->lv[l]; }
   size_t bytes() const { return bytes_; }
@@ -131,7 +131,8 @@ class TallGrid {
   TallRec* dev_rec_ = nullptr;
   float *in_u_ = nullptr, *in_v_ = nullptr, *in_w_ = nullptr;
   float *rm_in_ = nullptr, *rm_out_ = nullptr;  // remesh staging: phi, u, v, w in and out
-  int* rm_b_ = nullptr;                         // remesh bases (two buffers), flag, counter
+  int* rm_b_ = nullptr;                         // remesh counter, bases (two buffers)
+  int* rm_host_ = nullptr;                      // pinned: the counter and the new bases
   bool host_io_ = false;
   int id_ = 0;
   std::vector<void*> allocations_;

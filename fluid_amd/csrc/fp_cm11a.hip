@@ -350,65 +350,43 @@ __global__ void k_cm_residual(CmLevel L, const float* __restrict__ rhs, float* _
   }
 }
 
-// mgRestrictResidual (…multigrid.wgsl.ts:210-215)
-__global__ void k_cm_restrict(CmLevel F, const float* __restrict__ in, CmLevel C, float* __restrict__ out) {
-  CM_FOR(i, C.n) {
-    int X, Y, Z;
-    cdecode(C, i, X, Y, Z);
-    float t[8];
+// mgTrilinearPressure (…multigrid.wgsl.ts:217-241) at fine cell i
+__device__ __forceinline__ float trilinear(const CmLevel& C, const float* cp, const CmLevel& F, int i) {
+  int id[3];
+  cdecode(F, i, id[0], id[1], id[2]);
+  const int fd[3] = {F.D0, F.D1, F.D2}, cd[3] = {C.D0, C.D1, C.D2};
+  float f[3];
+  int base[3];
 #pragma unroll
-    for (int o = 0; o < 8; ++o) t[o] = in[fine_child(F, C, X, Y, Z, o)];
-    out[i] = d4s8(t) / 8.0f;
+  for (int a = 0; a < 3; ++a) {
+    const float fine_phys = (float)(fd[a] - 2), coarse_phys = (float)(cd[a] - 2);
+    const float scale = coarse_phys / fmaxf(fine_phys, 1.0f);
+    const float q = ((float)id[a] - 0.5f) * scale + 0.5f;
+    const float fl = floorf(q);
+    base[a] = (int)fl;
+    f[a] = q - fl;
   }
+  float values[8], weights[8];
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    const int ox = o & 1, oy = (o >> 1) & 1, oz = (o >> 2) & 1;
+    const int px = base[0] + ox, py = base[1] + oy, pz = base[2] + oz;
+    values[o] = 0.0f;
+    weights[o] = 0.0f;
+    if (!cinterior(C, px, py, pz)) continue;
+    const float w = ((ox ? f[0] : 1.0f - f[0]) * (oy ? f[1] : 1.0f - f[1])) * (oz ? f[2] : 1.0f - f[2]);
+    values[o] = w * cp[cidx(C, px, py, pz)];
+    weights[o] = w;
+  }
+  const float value = d4s8(values), total = d4s8(weights);
+  return total > 0.0f ? value / total : 0.0f;
 }
 
-// mgTrilinearPressure + mgProlongateAdd / Assign (…multigrid.wgsl.ts:217-253)
+// mgProlongateAdd / Assign (…multigrid.wgsl.ts:243-253)
 __global__ void k_cm_prolong(CmLevel C, CmLevel F, int add) {
   CM_FOR(i, F.n) {
-    int id[3];
-    cdecode(F, i, id[0], id[1], id[2]);
-    const int fd[3] = {F.D0, F.D1, F.D2}, cd[3] = {C.D0, C.D1, C.D2};
-    float f[3];
-    int base[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const float fine_phys = (float)(fd[a] - 2), coarse_phys = (float)(cd[a] - 2);
-      const float scale = coarse_phys / fmaxf(fine_phys, 1.0f);
-      const float q = ((float)id[a] - 0.5f) * scale + 0.5f;
-      const float fl = floorf(q);
-      base[a] = (int)fl;
-      f[a] = q - fl;
-    }
-    float values[8], weights[8];
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      const int ox = o & 1, oy = (o >> 1) & 1, oz = (o >> 2) & 1;
-      const int px = base[0] + ox, py = base[1] + oy, pz = base[2] + oz;
-      values[o] = 0.0f;
-      weights[o] = 0.0f;
-      if (!cinterior(C, px, py, pz)) continue;
-      const float w = ((ox ? f[0] : 1.0f - f[0]) * (oy ? f[1] : 1.0f - f[1])) * (oz ? f[2] : 1.0f - f[2]);
-      values[o] = w * C.p[cidx(C, px, py, pz)];
-      weights[o] = w;
-    }
-    const float value = d4s8(values), total = d4s8(weights);
-    const float t = total > 0.0f ? value / total : 0.0f;
+    const float t = trilinear(C, C.p, F, i);
     F.p[i] = add ? F.p[i] + t : t;
-  }
-}
-
-// mgDownsampleSubtract / mgDownsampleMinimum (…multigrid.wgsl.ts:311-323)
-__global__ void k_cm_down_min(CmLevel F, const float* __restrict__ fmin, int subtract, CmLevel C) {
-  CM_FOR(i, C.n) {
-    int X, Y, Z;
-    cdecode(C, i, X, Y, Z);
-    float lower = kNegBig;
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      const int j = fine_child(F, C, X, Y, Z, o);
-      lower = fmaxf(lower, subtract ? fmin[j] - F.p[j] : fmin[j]);
-    }
-    C.pmin[i] = lower;
   }
 }
 
@@ -451,12 +429,11 @@ __device__ __forceinline__ float coarse_coefficient(const CmLevel& L, int i, int
 
 // mgSolveCoarsest (…multigrid.wgsl.ts:404-471): one workgroup, a lane per
 // padded cell, double-single projected red-black sweeps in LDS until the
-// projected residual (1/s) is at most tol, or cap sweeps.
-__global__ __launch_bounds__(kCoarseLanes) void k_cm_coarse(CmLevel L, const float* __restrict__ rhs,
-                                                            const float* __restrict__ pmin, float dt, float rho,
-                                                            float tol, int cap, int open_top, CmStats* stats) {
-  __shared__ float sx[kCoarseLanes], sy[kCoarseLanes];
-  __shared__ unsigned s_max;
+// projected residual (1/s) is at most tol, or cap sweeps.  p, rhs and pmin may
+// lie in LDS.
+__device__ __forceinline__ void coarsest_solve(const CmLevel& L, float* p, const float* rhs, const float* pmin,
+                                               float dt, float rho, float tol, int cap, int open_top, CmStats* stats,
+                                               float* sx, float* sy, unsigned& s_max) {
   const int lane = threadIdx.x;
   const bool live = lane < L.n;
   int X = 0, Y = 0, Z = 0;
@@ -472,7 +449,7 @@ __global__ __launch_bounds__(kCoarseLanes) void k_cm_coarse(CmLevel L, const flo
     liquid = L.phi[lane] < 0.0f;
     r = rhs[lane];
     pm = pmin[lane];
-    sx[lane] = L.p[lane];
+    sx[lane] = p[lane];
     sy[lane] = 0.0f;
     if (liquid)
 #pragma unroll
@@ -544,13 +521,303 @@ __global__ __launch_bounds__(kCoarseLanes) void k_cm_coarse(CmLevel L, const flo
     }
     __syncthreads();  // s_max is reset by the next iteration
   }
-  if (live) L.p[lane] = sx[lane] + sy[lane];
+  if (live) p[lane] = sx[lane] + sy[lane];
   if (lane == 0) {
     stats->coarse_sweeps = max(stats->coarse_sweeps, iterations);
     stats->coarse_residual_bits = max(stats->coarse_residual_bits, __float_as_uint(worst));
     stats->coarse_failed += converged ? 0 : 1;
     stats->coarse_solves += 1;
   }
+}
+
+__global__ __launch_bounds__(kCoarseLanes) void k_cm_coarse(CmLevel L, const float* __restrict__ rhs,
+                                                            const float* __restrict__ pmin, float dt, float rho,
+                                                            float tol, int cap, int open_top, CmStats* stats) {
+  __shared__ float sx[kCoarseLanes], sy[kCoarseLanes];
+  __shared__ unsigned s_max;
+  coarsest_solve(L, L.p, rhs, pmin, dt, rho, tol, cap, open_top, stats, sx, sy, s_max);
+}
+
+// mgResidual, mgRestrictResidual (…multigrid.wgsl.ts:197-215), the zero start
+// and mgDownsampleSubtract (:311-323) of the next level in one launch: a lane per coarse cell evaluates the stencils of its
+// eight children (a child away from the halo belongs to one coarse cell, so
+// hardly any residual is made twice).
+__global__ void k_cm_descend(CmLevel F, const float* __restrict__ rhs, const float* __restrict__ fmin, int constrained,
+                             CmLevel C) {
+  CM_FOR(i, C.n) {
+    int X, Y, Z;
+    cdecode(C, i, X, Y, Z);
+    float t[8];
+    float lower = kNegBig;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const int j = fine_child(F, C, X, Y, Z, o);
+      const float4 own = F.coef[j];
+      if (constrained) lower = fmaxf(lower, fmin[j] - F.p[j]);
+      t[o] = 0.0f;
+      if (own.w > 0.5f) {
+        int x, y, z;
+        cdecode(F, j, x, y, z);
+        Stencil s;
+        stencil(F, j, x, y, z, own, s);
+        t[o] = rhs[j] - apply_at(F.p, j, s);
+      }
+    }
+    C.rhs0[i] = d4s8(t) / 8.0f;
+    C.p[i] = 0.0f;
+    C.pmin[i] = lower;
+  }
+}
+
+// mgRestrictResidual and mgDownsampleMinimum of a full cycle's way down
+__global__ void k_cm_full_down(CmLevel F, const float* __restrict__ fmin, int constrained, CmLevel C) {
+  CM_FOR(i, C.n) {
+    int X, Y, Z;
+    cdecode(C, i, X, Y, Z);
+    float t[8];
+    float lower = kNegBig;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const int j = fine_child(F, C, X, Y, Z, o);
+      t[o] = F.rhs1[j];
+      if (constrained) lower = fmaxf(lower, fmin[j]);
+    }
+    C.rhs1[i] = d4s8(t) / 8.0f;
+    C.pmin[i] = lower;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The tail of the schedule in one workgroup: every level from `first` on (at
+// most kTailCells padded cells in all) keeps its pressure, right-hand sides
+// and p_min in LDS, so a colour pass is a barrier instead of a launch.  On a
+// 64^3 grid 1152 of the 1560 colour passes are on these levels, and a launch
+// of one took 4 to 5 us with its gap; a V-cycle from 18^3 takes 82 us here, one
+// of 72 passes and 3 transfers, or about one us a pass.  A lane owns (even z, odd z) pairs of cells, one of each colour, and
+// holds their coefficients in registers for a whole smoothing leg.  The
+// arithmetic is that of k_cm_smooth, k_cm_residual, k_cm_restrict,
+// k_cm_down_min, k_cm_prolong and k_cm_coarse.
+// ---------------------------------------------------------------------------
+constexpr int kTailLanes = 1024;
+constexpr int kTailSlots = 3;       // pairs per lane on the first level
+constexpr int kTailCells = 7424;    // 16 bytes of LDS each, and 4 for the first level's residuals
+constexpr int kTailLevels = kMaxLevels;
+
+struct CmTail {
+  CmLevel lv[kTailLevels];
+  int first, levels, constraint_levels;
+  int sweeps;
+  float dt, rho, tol;
+  int cap, open_top;
+};
+
+template <int S>
+struct TailCells {
+  float a[2][S][6], diag[2][S], rhs[2][S], pm[2][S];
+  int i[2][S];             // LDS index, -1: no cell
+  unsigned liq[2][S];      // bits 0-5: the neighbour is liquid; bit 6: the cell is
+  __device__ __forceinline__ void load(const CmLevel& L, const float* rhs_, const float* pmin_) {
+    const int PZ = (L.D2 + 1) / 2, pairs = L.D0 * L.D1 * PZ;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int q = (int)threadIdx.x + kTailLanes * s;
+      const int pz = q % PZ, t = q / PZ, Y = t % L.D1, X = t / L.D1;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int Z = 2 * pz + ((X + Y + c) & 1);
+        const bool in = q < pairs && Z < L.D2;
+        const int j = in ? cidx(L, X, Y, Z) : 0;
+        i[c][s] = in ? j : -1;
+        liq[c][s] = 0;
+        const float4 own = L.coef[j];
+        rhs[c][s] = rhs_[j];
+        pm[c][s] = pmin_[j];
+        Stencil st;
+        stencil(L, j, in ? X : 0, in ? Y : 0, in ? Z : 0, own, st);
+#pragma unroll
+        for (int nb = 0; nb < 6; ++nb) {
+          a[c][s][nb] = st.a[nb];
+          liq[c][s] |= st.liq[nb] ? 1u << nb : 0u;
+        }
+        liq[c][s] |= own.w > 0.5f ? 64u : 0u;
+        diag[c][s] = d4s6(st.a);
+      }
+    }
+  }
+  __device__ __forceinline__ void neighbours(const CmLevel& L, const float* p, int c, int s, float* v) const {
+    const int off[6] = {-L.D1 * L.D2, L.D1 * L.D2, -L.D2, L.D2, -1, 1};
+#pragma unroll
+    for (int nb = 0; nb < 6; ++nb) {
+      const bool l = liq[c][s] >> nb & 1;
+      const float x = p[l ? i[c][s] + off[nb] : i[c][s]];
+      v[nb] = l ? x : 0.0f;
+    }
+  }
+  // mgSmoothColour of one colour
+  __device__ __forceinline__ void smooth(const CmLevel& L, float* p, int c) const {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (i[c][s] < 0) continue;
+      if (!(liq[c][s] & 64u)) {
+        p[i[c][s]] = fmaxf(p[i[c][s]], pm[c][s]);
+        continue;
+      }
+      float v[6], st[6];
+      neighbours(L, p, c, s, v);
+#pragma unroll
+      for (int nb = 0; nb < 6; ++nb) st[nb] = (liq[c][s] >> nb & 1) ? a[c][s][nb] * v[nb] : 0.0f;
+      const float sum = d4s6(st);
+      const float pn = diag[c][s] > 0.0f ? (sum + rhs[c][s]) / diag[c][s] : 0.0f;
+      p[i[c][s]] = fmaxf(pn, pm[c][s]);
+    }
+  }
+  __device__ __forceinline__ void residual(const CmLevel& L, const float* p, float* out) const {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (i[c][s] < 0) continue;
+        float r = 0.0f;
+        if (liq[c][s] & 64u) {
+          float v[6], t[6];
+          neighbours(L, p, c, s, v);
+          const float centre = p[i[c][s]];
+#pragma unroll
+          for (int nb = 0; nb < 6; ++nb) t[nb] = a[c][s][nb] * (centre - v[nb]);
+          r = rhs[c][s] - d4s6(t);
+        }
+        out[i[c][s]] = r;
+      }
+  }
+};
+
+// A level's arrays in LDS: p, rhs0, rhs1, pmin.
+struct TailArrays {
+  float *p, *rhs0, *rhs1, *pmin;
+};
+__device__ __forceinline__ TailArrays tail_arrays(const CmTail& T, float* base, int l) {
+  for (int k = T.first; k < l; ++k) base += 4 * T.lv[k].n;
+  const int n = T.lv[l].n;
+  return TailArrays{base, base + n, base + 2 * n, base + 3 * n};
+}
+
+template <int S>
+__device__ __forceinline__ void tail_smooth(const CmTail& T, int l, const TailArrays& A, const float* rhs, float* res) {
+  const CmLevel& L = T.lv[l];
+  TailCells<S> cells;
+  cells.load(L, rhs, A.pmin);
+  for (int k = 0; k < T.sweeps; ++k)
+    for (int c = 0; c < 2; ++c) {
+      cells.smooth(L, A.p, c);
+      __syncthreads();
+    }
+  if (res) {
+    cells.residual(L, A.p, res);
+    __syncthreads();
+  }
+}
+
+__device__ __forceinline__ void tail_prolong(const CmLevel& C, const float* cp, const CmLevel& F, float* fp, int add) {
+  for (int i = (int)threadIdx.x; i < F.n; i += kTailLanes) {
+    const float t = trilinear(C, cp, F, i);
+    fp[i] = add ? fp[i] + t : t;
+  }
+}
+
+// full: 1 the part of a full cycle on these levels (in: the first level's rhs1
+// and p_min; out: its pressure after its V-cycle), 0 one V-cycle from the
+// first level (in: its rhs0 and p_min, pressure zero).
+__global__ __launch_bounds__(kTailLanes) void k_cm_tail(CmTail T, int full, CmStats* stats) {
+  extern __shared__ float s_tail[];
+  __shared__ float sx[kCoarseLanes], sy[kCoarseLanes];
+  __shared__ unsigned s_max;
+  const int tid = (int)threadIdx.x, first = T.first, last = T.levels - 1;
+  float* res = s_tail;  // the first level's cells, reused by the levels below it
+  float* base = s_tail + T.lv[first].n;
+  {
+    const CmLevel& L = T.lv[first];
+    const TailArrays A = tail_arrays(T, base, first);
+    const float* __restrict__ src = full ? L.rhs1 : L.rhs0;
+    float* dst = full ? A.rhs1 : A.rhs0;
+    for (int i = tid; i < L.n; i += kTailLanes) {
+      A.p[i] = 0.0f;
+      dst[i] = src[i];
+      A.pmin[i] = L.pmin[i];
+    }
+  }
+  __syncthreads();
+  // one V-cycle from level l0 with its right-hand side
+  auto vcycle = [&](int l0, bool first_rhs1) {
+    for (int l = l0; l < last; ++l) {
+      const TailArrays A = tail_arrays(T, base, l), N = tail_arrays(T, base, l + 1);
+      const float* rhs = l == l0 && first_rhs1 ? A.rhs1 : A.rhs0;
+      if (l == first) tail_smooth<kTailSlots>(T, l, A, rhs, res);
+      else tail_smooth<1>(T, l, A, rhs, res);
+      const CmLevel &F = T.lv[l], &C = T.lv[l + 1];
+      for (int i = tid; i < C.n; i += kTailLanes) {
+        int X, Y, Z;
+        cdecode(C, i, X, Y, Z);
+        float t[8], lower = kNegBig;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          const int j = fine_child(F, C, X, Y, Z, o);
+          t[o] = res[j];
+          if (l < T.constraint_levels) lower = fmaxf(lower, A.pmin[j] - A.p[j]);
+        }
+        N.rhs0[i] = d4s8(t) / 8.0f;
+        N.p[i] = 0.0f;
+        N.pmin[i] = lower;
+      }
+      __syncthreads();
+    }
+    {
+      const TailArrays A = tail_arrays(T, base, last);
+      coarsest_solve(T.lv[last], A.p, l0 == last && first_rhs1 ? A.rhs1 : A.rhs0, A.pmin, T.dt, T.rho, T.tol, T.cap,
+                     T.open_top, stats, sx, sy, s_max);
+      __syncthreads();
+    }
+    for (int l = last - 1; l >= l0; --l) {
+      const TailArrays A = tail_arrays(T, base, l), N = tail_arrays(T, base, l + 1);
+      tail_prolong(T.lv[l + 1], N.p, T.lv[l], A.p, 1);
+      __syncthreads();
+      const float* rhs = l == l0 && first_rhs1 ? A.rhs1 : A.rhs0;
+      if (l == first) tail_smooth<kTailSlots>(T, l, A, rhs, nullptr);
+      else tail_smooth<1>(T, l, A, rhs, nullptr);
+    }
+  };
+  if (full) {
+    for (int l = first; l < last; ++l) {
+      const TailArrays A = tail_arrays(T, base, l), N = tail_arrays(T, base, l + 1);
+      const CmLevel &F = T.lv[l], &C = T.lv[l + 1];
+      for (int i = tid; i < C.n; i += kTailLanes) {
+        int X, Y, Z;
+        cdecode(C, i, X, Y, Z);
+        float t[8], lower = kNegBig;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          const int j = fine_child(F, C, X, Y, Z, o);
+          t[o] = A.rhs1[j];
+          if (l < T.constraint_levels) lower = fmaxf(lower, A.pmin[j]);
+        }
+        N.rhs1[i] = d4s8(t) / 8.0f;
+        N.p[i] = 0.0f;
+        N.pmin[i] = lower;
+      }
+      __syncthreads();
+    }
+    for (int l = last; l >= first; --l) {
+      if (l < last) {
+        tail_prolong(T.lv[l + 1], tail_arrays(T, base, l + 1).p, T.lv[l], tail_arrays(T, base, l).p, 0);
+        __syncthreads();
+      }
+      vcycle(l, true);
+    }
+  } else {
+    vcycle(first, false);
+  }
+  const CmLevel& L = T.lv[first];
+  const TailArrays A = tail_arrays(T, base, first);
+  for (int i = tid; i < L.n; i += kTailLanes) L.p[i] = A.p[i];
 }
 
 // mgMeasureFineResidual (…multigrid.wgsl.ts:473-481): max projected residual
@@ -732,7 +999,7 @@ size_t Cm11a::estimate_bytes(int nx, int ny, int nz) {
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   for (int l = 0; l < L; ++l) {
     const size_t n = (size_t)(dims[l][0] + 2) * (dims[l][1] + 2) * (dims[l][2] + 2);
-    total += 7 * up(n * 4) + 2 * up(n * 16);
+    total += 6 * up(n * 4) + 2 * up(n * 16);
     if (l == 0) total += 4 * up(n * 4);
   }
   return total + up((size_t)kMeasureBlocks * 16) + up(sizeof(CmStats));
@@ -781,7 +1048,6 @@ int Cm11a::create(int nx, int ny, int nz, double h) {
     if (!rc) rc = alloc((void**)&c.p, b4);
     if (!rc) rc = alloc((void**)&c.rhs0, b4);
     if (!rc) rc = alloc((void**)&c.rhs1, b4);
-    if (!rc) rc = alloc((void**)&c.res, b4);
     if (!rc) rc = alloc((void**)&c.pmin, b4);
     if (rc) return rc;
   }
@@ -792,7 +1058,19 @@ int Cm11a::create(int nx, int ny, int nz, double h) {
   if (!rc) rc = alloc((void**)&backup_, b0);
   if (!rc) rc = alloc((void**)&partials_, (size_t)kMeasureBlocks * 16);
   if (!rc) rc = alloc((void**)&stats_, sizeof(CmStats));
-  return rc;
+  if (rc) return rc;
+  // the tail starts at the first level (not the finest) whose levels fit; a
+  // device that gives a workgroup less LDS keeps one launch per pass
+  for (int l = 1; l + 1 < L && tail_ == 0; ++l) {
+    const size_t lds = tail_lds(l);
+    if (!lds) continue;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cm_tail), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) == hipSuccess)
+      tail_ = l;
+    else
+      (void)hipGetLastError();
+  }
+  return FP_OK;
 }
 
 void Cm11a::coarse_solve(hipStream_t s, const float* rhs, const float* pmin) {
@@ -800,6 +1078,36 @@ void Cm11a::coarse_solve(hipStream_t s, const float* rhs, const float* pmin) {
   const int threads = std::max(64, ((c.n + 63) / 64) * 64);
   hipLaunchKernelGGL(k_cm_coarse, dim3(1), dim3(threads), 0, s, c, rhs, pmin, dt_, rho_, tol_, cap_, open_top_,
                      stats_);
+}
+
+// Bytes of k_cm_tail's dynamic LDS for the levels from `first` on, 0 when they
+// do not fit its lanes and LDS.
+size_t Cm11a::tail_lds(int first) const {
+  const int L = (int)lv_.size();
+  long long cells = 0;
+  for (int l = first; l < L; ++l) cells += lv_[l].n;
+  auto pairs = [&](int l) { return (long long)lv_[l].D0 * lv_[l].D1 * ((lv_[l].D2 + 1) / 2); };
+  if (pairs(first) > (long long)kTailSlots * kTailLanes) return 0;
+  if (first + 1 < L - 1 && pairs(first + 1) > kTailLanes) return 0;
+  if (cells > kTailCells || L > kTailLevels) return 0;
+  return ((size_t)cells * 4 + (size_t)lv_[first].n) * sizeof(float);
+}
+
+void Cm11a::tail(hipStream_t s, int full) {
+  CmTail t;
+  std::memset(&t, 0, sizeof(t));
+  const int L = (int)lv_.size();
+  for (int l = 0; l < L; ++l) t.lv[l] = lv_[l];
+  t.first = tail_;
+  t.levels = L;
+  t.constraint_levels = constraint_levels_;
+  t.sweeps = pre_;
+  t.dt = dt_;
+  t.rho = rho_;
+  t.tol = tol_;
+  t.cap = cap_;
+  t.open_top = open_top_;
+  hipLaunchKernelGGL(k_cm_tail, dim3(1), dim3(kTailLanes), tail_lds(tail_), s, t, full, stats_);
 }
 
 // vCycle (…multigrid.ts:518-533); pmin0: the finest level's current p_min
@@ -814,14 +1122,9 @@ void Cm11a::vcycle(hipStream_t s, int l, const float* rhs, const float* pmin0) {
   CmLevel& d = lv_[l + 1];
   for (int i = 0; i < pre_; ++i)
     for (int colour = 0; colour < 2; ++colour) CM_LAUNCH(k_cm_smooth, c.n, s, c, rhs, pmin, colour);
-  CM_LAUNCH(k_cm_residual, c.n, s, c, rhs, c.res);
-  CM_LAUNCH(k_cm_restrict, d.n, s, c, (const float*)c.res, d, d.rhs0);
-  CM_LAUNCH(k_cm_fill, d.n, s, d.p, d.n, 0.0f);
-  if (l < constraint_levels_)
-    CM_LAUNCH(k_cm_down_min, d.n, s, c, pmin, 1, d);
-  else
-    CM_LAUNCH(k_cm_fill, d.n, s, d.pmin, d.n, kNegBig);
-  vcycle(s, l + 1, d.rhs0, pmin0);
+  CM_LAUNCH(k_cm_descend, d.n, s, c, rhs, pmin, l < constraint_levels_ ? 1 : 0, d);
+  if (l + 1 == tail_) tail(s, 0);
+  else vcycle(s, l + 1, d.rhs0, pmin0);
   CM_LAUNCH(k_cm_prolong, c.n, s, d, c, 1);
   for (int i = 0; i < post_; ++i)
     for (int colour = 0; colour < 2; ++colour) CM_LAUNCH(k_cm_smooth, c.n, s, c, rhs, pmin, colour);
@@ -833,19 +1136,18 @@ void Cm11a::full_cycle(hipStream_t s, const float* pmin0) {
   CmLevel& f = lv_[0];
   CM_LAUNCH(k_cm_backup_shift, f.n, s, (const float*)f.p, pmin0, backup_, pshift_, f.n);
   CM_LAUNCH(k_cm_residual, f.n, s, f, (const float*)b_, f.rhs1);
-  for (int l = 0; l + 1 < L; ++l) {
-    CmLevel& c = lv_[l];
-    CmLevel& d = lv_[l + 1];
-    CM_LAUNCH(k_cm_restrict, d.n, s, c, (const float*)c.rhs1, d, d.rhs1);
-    if (l < constraint_levels_)
-      CM_LAUNCH(k_cm_down_min, d.n, s, c, (const float*)(l == 0 ? pshift_ : c.pmin), 0, d);
-    else
-      CM_LAUNCH(k_cm_fill, d.n, s, d.pmin, d.n, kNegBig);
+  const int deep = tail_ > 0 ? tail_ : L - 1;  // the levels below run in the tail, or are the coarsest
+  for (int l = 0; l < deep; ++l)
+    CM_LAUNCH(k_cm_full_down, lv_[l + 1].n, s, lv_[l], (const float*)(l == 0 ? pshift_ : lv_[l].pmin),
+              l < constraint_levels_ ? 1 : 0, lv_[l + 1]);
+  if (tail_ > 0) {
+    tail(s, 1);
+  } else {
+    CmLevel& cc = lv_[L - 1];
+    CM_LAUNCH(k_cm_fill, cc.n, s, cc.p, cc.n, 0.0f);
+    coarse_solve(s, cc.rhs1, L == 1 ? pshift_ : cc.pmin);
   }
-  CmLevel& cc = lv_[L - 1];
-  CM_LAUNCH(k_cm_fill, cc.n, s, cc.p, cc.n, 0.0f);
-  coarse_solve(s, cc.rhs1, L == 1 ? pshift_ : cc.pmin);
-  for (int l = L - 2; l >= 0; --l) {
+  for (int l = deep - 1; l >= 0; --l) {
     CM_LAUNCH(k_cm_prolong, lv_[l].n, s, lv_[l + 1], lv_[l], 0);
     vcycle(s, l, lv_[l].rhs1, pshift_);
   }

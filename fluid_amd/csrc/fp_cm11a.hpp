@@ -32,7 +32,6 @@ struct CmLevel {
   float* p;
   float* rhs0;     // V-cycle right-hand side
   float* rhs1;     // full-cycle correction right-hand side
-  float* res;      // residual scratch
   float* pmin;     // p_min of the level
 };
 
@@ -62,11 +61,14 @@ class Cm11a {
   void vcycle(hipStream_t s, int l, const float* rhs, const float* pmin0);
   void full_cycle(hipStream_t s, const float* pmin0);
   void coarse_solve(hipStream_t s, const float* rhs, const float* pmin);
+  size_t tail_lds(int first) const;
+  void tail(hipStream_t s, int full);
   std::vector<CmLevel> lv_;
   std::vector<void*> allocations_;
   size_t bytes_ = 0;
   int nx_ = 0, ny_ = 0, nz_ = 0;
   double h_ = 0.0;
+  int tail_ = 0;            // first level of the one-workgroup tail (0: none)
   float* b_ = nullptr;      // finest right-hand side
   float* pmin0_ = nullptr;  // finest p_min
   float* pshift_ = nullptr; // finest p_min - p during a full cycle

@@ -1209,8 +1209,10 @@ static size_t bottom_lds_max() {
     const size_t want = (size_t)block > fixed ? (size_t)block - fixed : 0;
     if (want > kBottomLdsMax &&
         hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bottom_lds<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)want) != hipSuccess)
+                            (int)want) != hipSuccess) {
+      (void)hipGetLastError();
       return kBottomLdsMax;
+    }
     return want;
   }();
   return most;

@@ -3,9 +3,9 @@
 // Kernels restate lib/methods/uniform/webgpu-uniform-pressure-multigrid.wgsl.ts
 // (cited per kernel) and the schedule of …multigrid.ts:488-576.  Every level
 // is a halo-padded FP32 lattice in HBM, z fastest, with packed float4
-// dual volumes and coefficients (one 16-byte load per cell).  Red-black
-// passes run in place: a pass reads only the other colour and writes only its
-// own, which is what the reference's ping-pong textures compute.  The whole
+// dual volumes and coefficients (one 16-byte word per cell).  A colour pass reads only the
+// other colour, so a sweep of both is what the reference's ping-pong textures
+// compute, whether it goes from one buffer to another or in place.  The whole
 // file is compiled without floating-point contraction, and sums follow the
 // reference's D4 order, so results equal oracle/fp_oracle_cm11a.c bit for bit.
 #pragma clang fp contract(off)
@@ -269,84 +269,155 @@ __device__ __forceinline__ float coefficient_raw(const CmLevel& L, int i, int X,
   return vf / (h * h * theta);
 }
 
+// A cell's stencil: its six coefficients (mgCoefficient,
+// …multigrid.wgsl.ts:116-122), their sum and the liquid flags (bits 0-5 the
+// neighbours, bit 6 the cell).  The level stores the three positive faces and
+// the flags in one 16-byte word; the negative faces are the positive ones of
+// the cells behind, so a stencil is one word and three floats, and neither
+// those loads nor the neighbours' pressures wait for another.  (All six
+// coefficients in 32 bytes a cell took 47.0 ms for a 256^3 projection against
+// 43.7: memory bounds the sweeps there.)
+struct CmRecord {
+  float a[6], diag;
+  unsigned liq;
+};
+__device__ __forceinline__ CmRecord record_at(const CmLevel& L, int i, int X, int Y, int Z) {
+  const float4 own = L.coef[i];
+  const float* c = reinterpret_cast<const float*>(L.coef);
+  const bool hx = X > 0, hy = Y > 0, hz = Z > 0;
+  const float mx = c[4 * (size_t)(hx ? i - L.D1 * L.D2 : i)], my = c[4 * (size_t)(hy ? i - L.D2 : i) + 1],
+              mz = c[4 * (size_t)(hz ? i - 1 : i) + 2];
+  CmRecord r{{hx ? mx : 0.0f, own.x, hy ? my : 0.0f, own.y, hz ? mz : 0.0f, own.z}, 0.0f, __float_as_uint(own.w)};
+  r.diag = d4s6(r.a);
+  return r;
+}
+__device__ __forceinline__ CmRecord record_at(const CmLevel& L, int i) {
+  int X, Y, Z;
+  cdecode(L, i, X, Y, Z);
+  return record_at(L, i, X, Y, Z);
+}
+constexpr unsigned kSelfLiquid = 64u;
+
 // mgBakeCoefficients (…multigrid.wgsl.ts:302-309)
 __global__ void k_cm_bake(CmLevel L, int open_top) {
   CM_FOR(i, L.n) {
     int X, Y, Z;
     cdecode(L, i, X, Y, Z);
+    unsigned liq = L.phi[i] < 0.0f ? kSelfLiquid : 0u;
+#pragma unroll
+    for (int nb = 0; nb < 6; ++nb) {
+      const int x = X + kNb[nb][0], y = Y + kNb[nb][1], z = Z + kNb[nb][2];
+      if (cvalid(L, x, y, z) && L.phi[cidx(L, x, y, z)] < 0.0f) liq |= 1u << nb;
+    }
     L.coef[i] = make_float4(coefficient_raw(L, i, X, Y, Z, 0, open_top), coefficient_raw(L, i, X, Y, Z, 1, open_top),
-                            coefficient_raw(L, i, X, Y, Z, 2, open_top), L.phi[i] < 0.0f ? 1.0f : 0.0f);
+                            coefficient_raw(L, i, X, Y, Z, 2, open_top), __uint_as_float(liq));
   }
 }
 
-// The cell's six coefficients (mgCoefficient, …multigrid.wgsl.ts:116-122),
-// neighbour flags (mgBakedLiquid) and indices
-struct Stencil {
-  float a[6];
-  int j[6];
-  bool liq[6];
-};
-__device__ __forceinline__ void stencil(const CmLevel& L, int i, int X, int Y, int Z, const float4& own,
-                                        Stencil& s) {
+// The liquid neighbours' pressures of cell i (0 elsewhere)
+__device__ __forceinline__ void neighbour_pressures(const CmLevel& L, const float* p, int i, unsigned liq, float* v) {
+  const int off[6] = {-L.D1 * L.D2, L.D1 * L.D2, -L.D2, L.D2, -1, 1};
 #pragma unroll
   for (int nb = 0; nb < 6; ++nb) {
-    const int axis = nb / 2, x = X + kNb[nb][0], y = Y + kNb[nb][1], z = Z + kNb[nb][2];
-    const bool in = cvalid(L, x, y, z);
-    const int j = in ? cidx(L, x, y, z) : i;
-    s.j[nb] = j;
-    if (nb & 1) {
-      s.a[nb] = comp(own, axis);
-      s.liq[nb] = in && L.coef[j].w > 0.5f;
-    } else {
-      const float4 cq = in ? L.coef[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      s.a[nb] = comp(cq, axis);
-      s.liq[nb] = in && cq.w > 0.5f;
-    }
+    const bool l = liq >> nb & 1;
+    const float x = p[l ? i + off[nb] : i];
+    v[nb] = l ? x : 0.0f;
   }
 }
-__device__ __forceinline__ float apply_at(const float* __restrict__ p, int i, const Stencil& s) {
-  const float centre = p[i];
+// A p at a cell
+__device__ __forceinline__ float apply_record(const CmRecord& r, float centre, const float* v) {
   float terms[6];
 #pragma unroll
-  for (int nb = 0; nb < 6; ++nb) terms[nb] = s.a[nb] * (centre - (s.liq[nb] ? p[s.j[nb]] : 0.0f));
+  for (int nb = 0; nb < 6; ++nb) terms[nb] = r.a[nb] * (centre - v[nb]);
   return d4s6(terms);
 }
-
-// mgSmoothColour (…multigrid.wgsl.ts:325-344): the cells of one colour, in place
-__global__ void k_cm_smooth(CmLevel L, const float* __restrict__ rhs, const float* __restrict__ pmin, int colour) {
-  CM_FOR(i, L.n) {
-    int X, Y, Z;
-    cdecode(L, i, X, Y, Z);
-    if (((X + Y + Z) & 1) != colour) continue;
-    const float4 own = L.coef[i];
-    if (!(own.w > 0.5f)) {
-      L.p[i] = fmaxf(L.p[i], pmin[i]);
-      continue;
-    }
-    Stencil s;
-    stencil(L, i, X, Y, Z, own, s);
-    float st[6];
+// mgSmoothColour's value of a cell (…multigrid.wgsl.ts:325-344)
+__device__ __forceinline__ float smoothed(const float* a, float diag, unsigned liq, const float* v, float rhs,
+                                          float centre, float pmin) {
+  if (!(liq & kSelfLiquid)) return fmaxf(centre, pmin);
+  float st[6];
 #pragma unroll
-    for (int nb = 0; nb < 6; ++nb) st[nb] = s.liq[nb] ? s.a[nb] * L.p[s.j[nb]] : 0.0f;
-    const float diag = d4s6(s.a), sum = d4s6(st);
-    const float pn = diag > 0.0f ? (sum + rhs[i]) / diag : 0.0f;
-    L.p[i] = fmaxf(pn, pmin[i]);
+  for (int nb = 0; nb < 6; ++nb) st[nb] = (liq >> nb & 1) ? a[nb] * v[nb] : 0.0f;
+  const float sum = d4s6(st);
+  const float pn = diag > 0.0f ? (sum + rhs) / diag : 0.0f;
+  return fmaxf(pn, pmin);
+}
+
+// One red-black sweep of a level in one launch, from p into p2: a workgroup
+// takes an 8 x 8 x 16 tile, updates the first colour on the tile and its ring
+// from the old pressure, passes it through LDS and updates the second colour
+// of the tile, as (even z, odd z) pairs of one cell of each colour.  The ring
+// makes half the first-colour work twice, but a colour pass as a launch of its
+// own was only latency on these levels, with three loads waiting for each
+// other: a sweep of the 66^3 and 34^3 levels takes 7.0 us, its two passes took
+// 10.2 and a gap more.  At 256^3, where memory bounds it, a projection takes
+// 43.7 ms against 45.9.
+constexpr int kSweepX = 8, kSweepY = 8, kSweepZ = 16, kSweepLanes = 512;
+__global__ __launch_bounds__(kSweepLanes) void k_cm_sweep(CmLevel L, const float* __restrict__ rhs,
+                                                          const float* __restrict__ pmin) {
+  constexpr int WX = kSweepX + 2, WY = kSweepY + 2, WP = kSweepZ / 2 + 2;  // ring 1, one pair on either side in z
+  constexpr int NP = WX * WY * WP, S = (NP + kSweepLanes - 1) / kSweepLanes;
+  static_assert(kSweepX * kSweepY * kSweepZ / 2 == kSweepLanes, "a lane per second-colour cell of the tile");
+  __shared__ float s_first[NP];
+  const float* __restrict__ p = L.p;
+  float* __restrict__ out = L.p2;
+  const int tz = (L.D2 + kSweepZ - 1) / kSweepZ, ty = (L.D1 + kSweepY - 1) / kSweepY;
+  const int b = (int)blockIdx.x, x0 = b / (tz * ty) * kSweepX, y0 = b / tz % ty * kSweepY, z0 = b % tz * kSweepZ;
+  // first colour: slots of window pairs
+  int fi[S];
+  CmRecord fr[S];
+  float fv[S][6], frhs[S], fp[S], fmin_[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int q = (int)threadIdx.x + kSweepLanes * s;
+    const int wp = q % WP, t = q / WP, X = x0 - 1 + t / WY, Y = y0 - 1 + t % WY;
+    const int Z = z0 - 2 + 2 * wp + ((X + Y) & 1);
+    const bool in = q < NP && cvalid(L, X, Y, Z);
+    const int i = in ? cidx(L, X, Y, Z) : 0;
+    fi[s] = in ? i : -1;
+    fr[s] = record_at(L, i, in ? X : 0, in ? Y : 0, in ? Z : 0);
+    if (!in) fr[s].liq = 0;
+    frhs[s] = rhs[i];
+    fp[s] = p[i];
+    fmin_[s] = pmin[i];
+    neighbour_pressures(L, p, i, fr[s].liq, fv[s]);
   }
+  // second colour: this lane's cell of the tile
+  const int lp = (int)threadIdx.x % (kSweepZ / 2), lt = (int)threadIdx.x / (kSweepZ / 2);
+  const int lx = lt / kSweepY, ly = lt % kSweepY, X = x0 + lx, Y = y0 + ly, odd = (X + Y + 1) & 1;
+  const int Z = z0 + 2 * lp + odd;
+  const bool mine = cvalid(L, X, Y, Z);
+  const int i = mine ? cidx(L, X, Y, Z) : 0;
+  const CmRecord r = record_at(L, i, mine ? X : 0, mine ? Y : 0, mine ? Z : 0);
+  const float sr = rhs[i], sp = p[i], sm = pmin[i];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (fi[s] < 0) continue;
+    const int q = (int)threadIdx.x + kSweepLanes * s;
+    const float v = smoothed(fr[s].a, fr[s].diag, fr[s].liq, fv[s], frhs[s], fp[s], fmin_[s]);
+    s_first[q] = v;
+    const int wp = q % WP, t = q / WP, wx = t / WY, wy = t % WY;
+    if (wx >= 1 && wx <= kSweepX && wy >= 1 && wy <= kSweepY && wp >= 1 && wp <= kSweepZ / 2) out[fi[s]] = v;
+  }
+  __syncthreads();
+  if (!mine) return;
+  // every neighbour is a first-colour cell: the pair of the row beside this
+  // one, or this row's pair and the one before or after it
+  const int c = ((lx + 1) * WY + ly + 1) * WP + lp + 1;
+  const int at[6] = {c - WY * WP, c + WY * WP, c - WP, c + WP, odd ? c : c - 1, odd ? c + 1 : c};
+  float v[6];
+#pragma unroll
+  for (int nb = 0; nb < 6; ++nb) v[nb] = (r.liq >> nb & 1) ? s_first[at[nb]] : 0.0f;
+  out[i] = smoothed(r.a, r.diag, r.liq, v, sr, sp, sm);
 }
 
 // mgResidual (…multigrid.wgsl.ts:197-205)
 __global__ void k_cm_residual(CmLevel L, const float* __restrict__ rhs, float* __restrict__ out) {
   CM_FOR(i, L.n) {
-    const float4 own = L.coef[i];
-    if (!(own.w > 0.5f)) {
-      out[i] = 0.0f;
-      continue;
-    }
-    int X, Y, Z;
-    cdecode(L, i, X, Y, Z);
-    Stencil s;
-    stencil(L, i, X, Y, Z, own, s);
-    out[i] = rhs[i] - apply_at(L.p, i, s);
+    const CmRecord r = record_at(L, i);
+    float v[6];
+    neighbour_pressures(L, L.p, i, r.liq, v);
+    out[i] = (r.liq & kSelfLiquid) ? rhs[i] - apply_record(r, L.p[i], v) : 0.0f;
   }
 }
 
@@ -552,16 +623,12 @@ __global__ void k_cm_descend(CmLevel F, const float* __restrict__ rhs, const flo
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
       const int j = fine_child(F, C, X, Y, Z, o);
-      const float4 own = F.coef[j];
-      if (constrained) lower = fmaxf(lower, fmin[j] - F.p[j]);
-      t[o] = 0.0f;
-      if (own.w > 0.5f) {
-        int x, y, z;
-        cdecode(F, j, x, y, z);
-        Stencil s;
-        stencil(F, j, x, y, z, own, s);
-        t[o] = rhs[j] - apply_at(F.p, j, s);
-      }
+      const CmRecord r = record_at(F, j);
+      const float centre = F.p[j];
+      if (constrained) lower = fmaxf(lower, fmin[j] - centre);
+      float v[6];
+      neighbour_pressures(F, F.p, j, r.liq, v);
+      t[o] = (r.liq & kSelfLiquid) ? rhs[j] - apply_record(r, centre, v) : 0.0f;
     }
     C.rhs0[i] = d4s8(t) / 8.0f;
     C.p[i] = 0.0f;
@@ -592,11 +659,11 @@ __global__ void k_cm_full_down(CmLevel F, const float* __restrict__ fmin, int co
 // most kTailCells padded cells in all) keeps its pressure, right-hand sides
 // and p_min in LDS, so a colour pass is a barrier instead of a launch.  On a
 // 64^3 grid 1152 of the 1560 colour passes are on these levels, and a launch
-// of one took 4 to 5 us with its gap; a V-cycle from 18^3 takes 82 us here, one
+// of one took 4 to 5 us with its gap; a V-cycle from 18^3 takes 63 us here, one
 // of 72 passes and 3 transfers, or about one us a pass.  A lane owns (even z, odd z) pairs of cells, one of each colour, and
 // holds their coefficients in registers for a whole smoothing leg.  The
-// arithmetic is that of k_cm_smooth, k_cm_residual, k_cm_restrict,
-// k_cm_down_min, k_cm_prolong and k_cm_coarse.
+// arithmetic is that of k_cm_sweep, k_cm_descend, k_cm_full_down, k_cm_prolong
+// and k_cm_coarse.
 // ---------------------------------------------------------------------------
 constexpr int kTailLanes = 1024;
 constexpr int kTailSlots = 3;       // pairs per lane on the first level
@@ -613,9 +680,9 @@ struct CmTail {
 
 template <int S>
 struct TailCells {
-  float a[2][S][6], diag[2][S], rhs[2][S], pm[2][S];
+  CmRecord r[2][S];
+  float rhs[2][S], pm[2][S];
   int i[2][S];             // LDS index, -1: no cell
-  unsigned liq[2][S];      // bits 0-5: the neighbour is liquid; bit 6: the cell is
   __device__ __forceinline__ void load(const CmLevel& L, const float* rhs_, const float* pmin_) {
     const int PZ = (L.D2 + 1) / 2, pairs = L.D0 * L.D1 * PZ;
 #pragma unroll
@@ -628,29 +695,10 @@ struct TailCells {
         const bool in = q < pairs && Z < L.D2;
         const int j = in ? cidx(L, X, Y, Z) : 0;
         i[c][s] = in ? j : -1;
-        liq[c][s] = 0;
-        const float4 own = L.coef[j];
+        r[c][s] = record_at(L, j, in ? X : 0, in ? Y : 0, in ? Z : 0);
         rhs[c][s] = rhs_[j];
         pm[c][s] = pmin_[j];
-        Stencil st;
-        stencil(L, j, in ? X : 0, in ? Y : 0, in ? Z : 0, own, st);
-#pragma unroll
-        for (int nb = 0; nb < 6; ++nb) {
-          a[c][s][nb] = st.a[nb];
-          liq[c][s] |= st.liq[nb] ? 1u << nb : 0u;
-        }
-        liq[c][s] |= own.w > 0.5f ? 64u : 0u;
-        diag[c][s] = d4s6(st.a);
       }
-    }
-  }
-  __device__ __forceinline__ void neighbours(const CmLevel& L, const float* p, int c, int s, float* v) const {
-    const int off[6] = {-L.D1 * L.D2, L.D1 * L.D2, -L.D2, L.D2, -1, 1};
-#pragma unroll
-    for (int nb = 0; nb < 6; ++nb) {
-      const bool l = liq[c][s] >> nb & 1;
-      const float x = p[l ? i[c][s] + off[nb] : i[c][s]];
-      v[nb] = l ? x : 0.0f;
     }
   }
   // mgSmoothColour of one colour
@@ -658,17 +706,9 @@ struct TailCells {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       if (i[c][s] < 0) continue;
-      if (!(liq[c][s] & 64u)) {
-        p[i[c][s]] = fmaxf(p[i[c][s]], pm[c][s]);
-        continue;
-      }
-      float v[6], st[6];
-      neighbours(L, p, c, s, v);
-#pragma unroll
-      for (int nb = 0; nb < 6; ++nb) st[nb] = (liq[c][s] >> nb & 1) ? a[c][s][nb] * v[nb] : 0.0f;
-      const float sum = d4s6(st);
-      const float pn = diag[c][s] > 0.0f ? (sum + rhs[c][s]) / diag[c][s] : 0.0f;
-      p[i[c][s]] = fmaxf(pn, pm[c][s]);
+      float v[6];
+      neighbour_pressures(L, p, i[c][s], r[c][s].liq, v);
+      p[i[c][s]] = smoothed(r[c][s].a, r[c][s].diag, r[c][s].liq, v, rhs[c][s], p[i[c][s]], pm[c][s]);
     }
   }
   __device__ __forceinline__ void residual(const CmLevel& L, const float* p, float* out) const {
@@ -677,16 +717,9 @@ struct TailCells {
 #pragma unroll
       for (int s = 0; s < S; ++s) {
         if (i[c][s] < 0) continue;
-        float r = 0.0f;
-        if (liq[c][s] & 64u) {
-          float v[6], t[6];
-          neighbours(L, p, c, s, v);
-          const float centre = p[i[c][s]];
-#pragma unroll
-          for (int nb = 0; nb < 6; ++nb) t[nb] = a[c][s][nb] * (centre - v[nb]);
-          r = rhs[c][s] - d4s6(t);
-        }
-        out[i[c][s]] = r;
+        float v[6];
+        neighbour_pressures(L, p, i[c][s], r[c][s].liq, v);
+        out[i[c][s]] = (r[c][s].liq & kSelfLiquid) ? rhs[c][s] - apply_record(r[c][s], p[i[c][s]], v) : 0.0f;
       }
   }
 };
@@ -820,6 +853,14 @@ __global__ __launch_bounds__(kTailLanes) void k_cm_tail(CmTail T, int full, CmSt
   for (int i = tid; i < L.n; i += kTailLanes) L.p[i] = A.p[i];
 }
 
+// Max of non-negative floats (as bits) into *out: one atomic per workgroup, and
+// only where it can raise the value.  One per wave on a single address, 4096
+// of them at 64^3, was 48 us of a 4 us pass.
+__device__ __forceinline__ void max_bits(float v, unsigned* out) {
+  const unsigned m = __float_as_uint(block_max(v));
+  if (threadIdx.x == 0 && m > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, m);
+}
+
 // mgMeasureFineResidual (…multigrid.wgsl.ts:473-481): max projected residual
 // (1/s) and, per workgroup, the sum of squares of the projected residual and
 // of b (the relative LCP residual of the report)
@@ -828,15 +869,13 @@ __global__ void k_cm_measure(CmLevel L, const float* __restrict__ b, const float
   double acc[2] = {0.0, 0.0};
   float mx = 0.0f;
   CM_FOR(i, L.n) {
-    const float4 own = L.coef[i];
-    if (!(own.w > 0.5f)) continue;
-    int X, Y, Z;
-    cdecode(L, i, X, Y, Z);
-    Stencil s;
-    stencil(L, i, X, Y, Z, own, s);
-    const float diag = d4s6(s.a);
+    const CmRecord c = record_at(L, i);
+    if (!(c.liq & kSelfLiquid)) continue;
+    const float diag = c.diag;
     if (diag <= 0.0f) continue;
-    const float r = b[i] - apply_at(L.p, i, s);
+    float v[6];
+    neighbour_pressures(L, L.p, i, c.liq, v);
+    const float r = b[i] - apply_record(c, L.p[i], v);
     const float gap = fmaxf(0.0f, L.p[i] - pmin[i]);
     const bool projects = r < 0.0f && -r >= gap * diag;
     const float pr = projects ? gap * diag : fabsf(r);
@@ -844,8 +883,7 @@ __global__ void k_cm_measure(CmLevel L, const float* __restrict__ b, const float
     acc[0] += (double)pr * (double)pr;
     acc[1] += (double)b[i] * (double)b[i];
   }
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) atomicMax(&stats->lcp_residual_bits, __float_as_uint(mx));
+  max_bits(mx, &stats->lcp_residual_bits);
   block_sum<2>(acc);
   if (threadIdx.x == 0) {
     partials[2 * blockIdx.x] = acc[0];
@@ -884,8 +922,7 @@ __global__ void k_cm_max_div(int nx, int ny, int nz, float h, const float* __res
     }
     mx = fmaxf(mx, fabsf(d4s6(terms)));
   }
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) atomicMax(out_bits, __float_as_uint(mx));
+  max_bits(mx, out_bits);
 }
 
 // project (webgpu-uniform-reference.wgsl.ts:1052-1099) on a box container:
@@ -999,7 +1036,7 @@ size_t Cm11a::estimate_bytes(int nx, int ny, int nz) {
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   for (int l = 0; l < L; ++l) {
     const size_t n = (size_t)(dims[l][0] + 2) * (dims[l][1] + 2) * (dims[l][2] + 2);
-    total += 6 * up(n * 4) + 2 * up(n * 16);
+    total += 7 * up(n * 4) + 2 * up(n * 16);
     if (l == 0) total += 4 * up(n * 4);
   }
   return total + up((size_t)kMeasureBlocks * 16) + up(sizeof(CmStats));
@@ -1046,6 +1083,7 @@ int Cm11a::create(int nx, int ny, int nz, double h) {
     if (!rc) rc = alloc((void**)&c.topo, b16);
     if (!rc) rc = alloc((void**)&c.coef, b16);
     if (!rc) rc = alloc((void**)&c.p, b4);
+    if (!rc) rc = alloc((void**)&c.p2, b4);
     if (!rc) rc = alloc((void**)&c.rhs0, b4);
     if (!rc) rc = alloc((void**)&c.rhs1, b4);
     if (!rc) rc = alloc((void**)&c.pmin, b4);
@@ -1110,6 +1148,17 @@ void Cm11a::tail(hipStream_t s, int full) {
   hipLaunchKernelGGL(k_cm_tail, dim3(1), dim3(kTailLanes), tail_lds(tail_), s, t, full, stats_);
 }
 
+// `count` red-black sweeps; each writes the level's other pressure buffer,
+// which then is the level's pressure.
+void Cm11a::sweeps(hipStream_t s, CmLevel& c, int count, const float* rhs, const float* pmin) {
+  auto tiles = [](int n, int t) { return (n + t - 1) / t; };
+  const int groups = tiles(c.D0, kSweepX) * tiles(c.D1, kSweepY) * tiles(c.D2, kSweepZ);
+  for (int i = 0; i < count; ++i) {
+    hipLaunchKernelGGL(k_cm_sweep, dim3(groups), dim3(kSweepLanes), 0, s, c, rhs, pmin);
+    std::swap(c.p, c.p2);
+  }
+}
+
 // vCycle (…multigrid.ts:518-533); pmin0: the finest level's current p_min
 void Cm11a::vcycle(hipStream_t s, int l, const float* rhs, const float* pmin0) {
   const int L = (int)lv_.size();
@@ -1120,14 +1169,12 @@ void Cm11a::vcycle(hipStream_t s, int l, const float* rhs, const float* pmin0) {
     return;
   }
   CmLevel& d = lv_[l + 1];
-  for (int i = 0; i < pre_; ++i)
-    for (int colour = 0; colour < 2; ++colour) CM_LAUNCH(k_cm_smooth, c.n, s, c, rhs, pmin, colour);
+  sweeps(s, c, pre_, rhs, pmin);
   CM_LAUNCH(k_cm_descend, d.n, s, c, rhs, pmin, l < constraint_levels_ ? 1 : 0, d);
   if (l + 1 == tail_) tail(s, 0);
   else vcycle(s, l + 1, d.rhs0, pmin0);
   CM_LAUNCH(k_cm_prolong, c.n, s, d, c, 1);
-  for (int i = 0; i < post_; ++i)
-    for (int colour = 0; colour < 2; ++colour) CM_LAUNCH(k_cm_smooth, c.n, s, c, rhs, pmin, colour);
+  sweeps(s, c, post_, rhs, pmin);
 }
 
 // fullCycle (…multigrid.ts:534-557)

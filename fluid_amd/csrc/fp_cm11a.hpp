@@ -28,8 +28,9 @@ struct CmLevel {
   float* phi_raw;  // coarsened level set (the raw pyramid)
   float* phi;      // continued one cell into the walls
   float4* topo;    // cell dual volume, +x/+y/+z face dual volumes
-  float4* coef;    // +x/+y/+z coefficients V / (h^2 theta), liquid flag
-  float* p;
+  float4* coef;    // +x/+y/+z coefficients V / (h^2 theta), liquid flags of the cell and its neighbours
+  float* p;        // pressure
+  float* p2;       // the buffer that the next sweep writes (they then change places)
   float* rhs0;     // V-cycle right-hand side
   float* rhs1;     // full-cycle correction right-hand side
   float* pmin;     // p_min of the level
@@ -61,6 +62,7 @@ class Cm11a {
   void vcycle(hipStream_t s, int l, const float* rhs, const float* pmin0);
   void full_cycle(hipStream_t s, const float* pmin0);
   void coarse_solve(hipStream_t s, const float* rhs, const float* pmin);
+  void sweeps(hipStream_t s, CmLevel& c, int count, const float* rhs, const float* pmin);
   size_t tail_lds(int first) const;
   void tail(hipStream_t s, int full);
   std::vector<CmLevel> lv_;

@@ -23,7 +23,8 @@ namespace fp {
 struct ExState {
   float* val[3];
   float* dist[3];
-  uint8_t* flags;  // bits 0-2 known(c), 3-5 active(c)
+  uint8_t* flags;  // bits 0-2 known(c)
+  uint8_t* stat;   // bits 2c, 2c+1: the face's part in the front (kQuiet ...)
 };
 
 // One level of the far-field hierarchy.
@@ -36,12 +37,21 @@ struct ExLevel {
   uint8_t* up_known;
 };
 
+// Counters are spread over kExSpread cache lines by workgroup: thousands of
+// atomics on one address take about 11 ns each.
+constexpr int kExSpread = 16;
 struct ExCounters {
-  int active[20];                  // [0] after the seed, [k] after pass k
-  int latest;                      // side holding the band result
-  int list_count;                  // cells of the band list
-  unsigned long long unknown;      // open faces left unknown
-  unsigned long long band_known;   // faces known after the band
+  int active[20][kExSpread][16];                     // [0] the seed's, [k] before pass k + 1
+  unsigned long long unknown[kExSpread][8];          // open faces left unknown
+  unsigned long long band_known[kExSpread][8];       // faces known after the band
+  int latest;                                        // side holding the band result
+  int list_count;                                    // cells of the band list
+};
+
+// Their sums, for the host.
+struct ExTotals {
+  int active[20];
+  unsigned long long unknown, band_known;
 };
 
 class Extrapolator {
@@ -72,6 +82,7 @@ class Extrapolator {
   int* list_ = nullptr;
   float* in_ = nullptr;  // host-memory staging: phi or density, u, v, w
   ExCounters* counters_ = nullptr;
+  ExTotals* totals_ = nullptr;
 };
 
 }  // namespace fp

@@ -180,85 +180,154 @@ __global__ __launch_bounds__(kThreads) void k_ex_classify(ExGeo g, const float* 
   }
 }
 
-// bits 0-2 open(c), 3-5 source(c)
-__device__ __forceinline__ unsigned cls_at(const ExGeo& g, const uint8_t* cls, int x, int y, int z) {
-  return ein(g.d, x, y, z) ? cls[eidx(g, x, y, z)] : 0u;
-}
-
-// the byte of each 6-neighbour (0 outside the domain), loaded without branches
-__device__ __forceinline__ void load6(const ExGeo& g, const uint8_t* __restrict__ a, unsigned i, int x, int y, int z,
-                                      unsigned* out) {
-  const unsigned sx = (unsigned)g.d[1] * g.d[2], sy = (unsigned)g.d[2];
-  const bool ok[6] = {x > 0, x + 1 < g.d[0], y > 0, y + 1 < g.d[1], z > 0, z + 1 < g.d[2]};
-  const unsigned idx[6] = {ok[0] ? i - sx : i, ok[1] ? i + sx : i, ok[2] ? i - sy : i,
-                           ok[3] ? i + sy : i, ok[4] ? i - 1 : i,  ok[5] ? i + 1 : i};
+// ---- four cells in a word ----
+// The byte arrays (classes, candidates) are worked on four consecutive cells
+// to a lane: the cells' bytes are one word and so are those of each neighbour
+// offset, loaded unaligned, with the bytes of cells that have no neighbour
+// there masked off.  Seven word loads serve four cells where a load per byte
+// took twenty-eight (the dilations and the seed were bound by them: at 384^3
+// the dilations take 32 to 69 us for 62 to 100, the seed, which also writes
+// less, 198 for 650).  A quad may run over a row's or a plane's end, so
+// nothing depends on the row length; the arrays carry quad_pad bytes on either
+// side for the words that reach past the grid.
+struct Quad {
+  unsigned i;         // first cell
+  unsigned in;        // mask of the cells below n
+  unsigned ok[6];     // mask of the cells that have the neighbour (-x, +x, -y, +y, -z, +z)
+  int x, y, z;        // of the first cell
+  bool row;           // the cells are one row's
+  __device__ __forceinline__ Quad(const ExGeo& g, unsigned n) {
+    const unsigned per_group = kThreads * 4;
+    i = chunk_of((n + per_group - 1) / per_group) * per_group + 4 * threadIdx.x;
+    in = 0;
+    row = false;
 #pragma unroll
-  for (int k = 0; k < 6; ++k) out[k] = a[idx[k]];
+    for (int k = 0; k < 6; ++k) ok[k] = 0;
+    if (i >= n) return;
+    edecode(g, i, x, y, z);
+    row = z + 3 < g.d[2];
+    if (row) {  // (so every cell is below n)
+      in = ~0u;
+      ok[0] = x > 0 ? ~0u : 0u;
+      ok[1] = x + 1 < g.d[0] ? ~0u : 0u;
+      ok[2] = y > 0 ? ~0u : 0u;
+      ok[3] = y + 1 < g.d[1] ? ~0u : 0u;
+      ok[4] = z > 0 ? ~0u : ~0u << 8;
+      ok[5] = z + 4 < g.d[2] ? ~0u : ~0u >> 8;
+      return;
+    }
+    int a = x, b = y, c = z;
 #pragma unroll
-  for (int k = 0; k < 6; ++k) out[k] = ok[k] ? out[k] : 0u;
+    for (int j = 0; j < 4; ++j) {
+      const unsigned m = i + j < n ? 0xffu << 8 * j : 0u;
+      in |= m;
+      ok[0] |= a > 0 ? m : 0u;
+      ok[1] |= a + 1 < g.d[0] ? m : 0u;
+      ok[2] |= b > 0 ? m : 0u;
+      ok[3] |= b + 1 < g.d[1] ? m : 0u;
+      ok[4] |= c > 0 ? m : 0u;
+      ok[5] |= c + 1 < g.d[2] ? m : 0u;
+      if (++c == g.d[2]) {
+        c = 0;
+        if (++b == g.d[1]) {
+          b = 0;
+          ++a;
+        }
+      }
+    }
+  }
+};
+__device__ __forceinline__ unsigned word_at(const uint8_t* p, int i) {
+  unsigned w;
+  __builtin_memcpy(&w, p + i, 4);
+  return w;
 }
+// the OR of the six neighbours' bytes, per cell
+__device__ __forceinline__ unsigned around(const ExGeo& g, const Quad& q, const uint8_t* __restrict__ a) {
+  const int sx = g.d[1] * g.d[2], sy = g.d[2], i = (int)q.i;
+  const int off[6] = {-sx, sx, -sy, sy, -1, 1};
+  unsigned w[6], m = 0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) w[k] = word_at(a, i + off[k]);
+#pragma unroll
+  for (int k = 0; k < 6; ++k) m |= w[k] & q.ok[k];
+  return m;
+}
+constexpr unsigned kBits3 = 0x07070707u, kBit = 0x01010101u;
 
-// seedActiveFront (…extrapolation.wgsl.ts:148-170).  Side A everywhere; side
-// B only where a pass can read it before writing it: the band list's cells
-// and their 6-neighbours, all within one cell of the last candidate
-// dilation (near: that mask; a pass writes every list cell of its
-// destination side, and reads its source side at list cells and their
-// neighbours only).
+// seedActiveFront (…extrapolation.wgsl.ts:148-170).  Flags everywhere; the
+// rest only where it is read: a known face's value (the hierarchy selects by
+// the flags), and the whole state, on both sides, where a pass can read it
+// before writing it: the band list's cells (listed) and their 6-neighbours (a
+// pass writes every list cell of its destination side, and reads its source
+// side at list cells and their neighbours only).  At 384^3 the list holds 1% of
+// the cells: inside the liquid the seed copies 12 bytes a cell, in the air
+// beyond the band it writes one, where it wrote 25 and 50.
 __global__ __launch_bounds__(kThreads) void k_ex_seed(ExGeo g, const uint8_t* __restrict__ cls,
-                                                     const uint8_t* __restrict__ near,
+                                                     const uint8_t* __restrict__ listed,
                                                      const float* __restrict__ u, const float* __restrict__ v,
                                                      const float* __restrict__ w, ExState a, ExState b,
                                                      ExCounters* cnt, unsigned n) {
-  unsigned me[kCells], nb[kCells][6], nr[kCells];
-  float in[kCells][3];
-#pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = min(cell_of(n, j), n - 1);
-    int x, y, z;
-    edecode(g, i, x, y, z);
-    me[j] = cls[i];
-    load6(g, cls, i, x, y, z, nb[j]);
-    unsigned m6[6];
-    load6(g, near, i, x, y, z, m6);
-    nr[j] = near[i] | m6[0] | m6[1] | m6[2] | m6[3] | m6[4] | m6[5];
-    // the positive face of every cell exists in the face arrays
-    in[j][0] = u[face_of(g, 0, x, y, z)];
-    in[j][1] = v[face_of(g, 1, x, y, z)];
-    in[j][2] = w[face_of(g, 2, x, y, z)];
-  }
+  const Quad q(g, n);
   int active = 0;
+  if (q.in) {
+    const unsigned me = word_at(cls, (int)q.i) & q.in;
+    const unsigned nr = (word_at(listed, (int)q.i) | around(g, q, listed)) & q.in;
+    const unsigned open = me & kBits3, known = me >> 3 & kBits3;
+    const unsigned act = open & ~known & (around(g, q, cls) >> 3 & kBits3);
+    const unsigned stat = (act & kBit) << 1 | (act >> 1 & kBit) << 3 | (act >> 2 & kBit) << 5;
+    static_assert(kActive == 2, "an active face's state is the upper of its two bits");
+    active = __popc(act);
+    reinterpret_cast<unsigned*>(a.flags)[q.i >> 2] = known;
+    if (nr) {
+      reinterpret_cast<unsigned*>(a.stat)[q.i >> 2] = stat;
+      reinterpret_cast<unsigned*>(b.flags)[q.i >> 2] = known;
+      reinterpret_cast<unsigned*>(b.stat)[q.i >> 2] = stat;
+    }
+    if (known || nr) {
+      // the positive face of every cell exists in the face arrays, four of a
+      // row side by side
+      float in[3][4], val[3][4], dist[3][4];
+      if (q.row) {
+        __builtin_memcpy(in[0], u + face_of(g, 0, q.x, q.y, q.z), 16);
+        __builtin_memcpy(in[1], v + face_of(g, 1, q.x, q.y, q.z), 16);
+        __builtin_memcpy(in[2], w + face_of(g, 2, q.x, q.y, q.z), 16);
+      } else {
+        int x = q.x, y = q.y, z = q.z;
 #pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = cell_of(n, j);
-    if (i >= n) break;
-    unsigned srcnb = 0;  // per component: a 6-neighbour is a source
-    for (int k = 0; k < 6; ++k) srcnb |= nb[j][k];
-    srcnb >>= 3;
-    unsigned flags = 0, stat = 0;
-    for (int c = 0; c < 3; ++c) {
-      float val = 0.0f, dist = kInf;
-      if (me[j] >> c & 1) {
-        if (me[j] >> (3 + c) & 1) {
-          val = in[j][c];
-          dist = 0.0f;
-          flags |= 1u << c;
-        } else if (srcnb >> c & 1) {
-          stat |= kActive << 2 * c;
-          active += 1;
+        for (int j = 0; j < 4; ++j) {
+          const bool there = q.in >> 8 * j & 1u;
+          in[0][j] = there ? u[face_of(g, 0, x, y, z)] : 0.0f;
+          in[1][j] = there ? v[face_of(g, 1, x, y, z)] : 0.0f;
+          in[2][j] = there ? w[face_of(g, 2, x, y, z)] : 0.0f;
+          if (++z == g.d[2]) {
+            z = 0;
+            if (++y == g.d[1]) {
+              y = 0;
+              ++x;
+            }
+          }
         }
       }
-      a.val[c][i] = val;
-      a.dist[c][i] = dist;
-      if (nr[j]) {
-        b.val[c][i] = val;
-        b.dist[c][i] = dist;
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool k = known >> (8 * j + c) & 1u;
+          val[c][j] = k ? in[c][j] : 0.0f;
+          dist[c][j] = k ? 0.0f : kInf;
+        }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float4 vc = make_float4(val[c][0], val[c][1], val[c][2], val[c][3]);
+        const float4 dc = make_float4(dist[c][0], dist[c][1], dist[c][2], dist[c][3]);
+        reinterpret_cast<float4*>(a.val[c])[q.i >> 2] = vc;
+        if (nr) {
+          reinterpret_cast<float4*>(a.dist[c])[q.i >> 2] = dc;
+          reinterpret_cast<float4*>(b.val[c])[q.i >> 2] = vc;
+          reinterpret_cast<float4*>(b.dist[c])[q.i >> 2] = dc;
+        }
       }
-    }
-    a.flags[i] = (uint8_t)flags;
-    a.stat[i] = (uint8_t)stat;
-    if (nr[j]) {
-      b.flags[i] = (uint8_t)flags;
-      b.stat[i] = (uint8_t)stat;
     }
   }
   const int s = block_sum(active);
@@ -267,32 +336,24 @@ __global__ __launch_bounds__(kThreads) void k_ex_seed(ExGeo g, const uint8_t* __
 
 // one 6-neighbour OR of the candidate bits; the last one appends the cells
 // with an open non-source candidate face to the band list (one atomic per
-// workgroup) and also stores its mask (the seed's near set)
+// workgroup) and stores which they are
 __global__ __launch_bounds__(kThreads) void k_ex_dilate(ExGeo g, const uint8_t* __restrict__ cls,
                                                        const uint8_t* __restrict__ in, uint8_t* __restrict__ out,
                                                        int last, int* __restrict__ list, ExCounters* cnt,
                                                        unsigned n) {
-  unsigned m[kCells], me[kCells];
-#pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = min(cell_of(n, j), n - 1);
-    int x, y, z;
-    edecode(g, i, x, y, z);
-    unsigned nb[6];
-    load6(g, in, i, x, y, z, nb);
-    m[j] = in[i] | nb[0] | nb[1] | nb[2] | nb[3] | nb[4] | nb[5];
-    me[j] = last ? cls[i] : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = cell_of(n, j);
-    if (i < n) out[i] = (uint8_t)m[j];
+  const Quad q(g, n);
+  unsigned takes = 0;
+  if (q.in) {
+    const unsigned me = last ? word_at(cls, (int)q.i) : 0u;
+    unsigned m = (word_at(in, (int)q.i) | around(g, q, in)) & q.in;
+    if (last) {
+      takes = m & me & ~(me >> 3) & kBits3;
+      takes = (takes | takes >> 1 | takes >> 2) & kBit;
+      m = takes;
+    }
+    reinterpret_cast<unsigned*>(out)[q.i >> 2] = m;
   }
   if (!last) return;
-  unsigned takes = 0;
-#pragma unroll
-  for (int j = 0; j < kCells; ++j)
-    if (cell_of(n, j) < n && (m[j] & (me[j] & 7u) & ~(me[j] >> 3)) != 0) takes |= 1u << j;
   int total;
   int at = block_scan(__popc(takes), &total);
   __shared__ int base;
@@ -300,8 +361,8 @@ __global__ __launch_bounds__(kThreads) void k_ex_dilate(ExGeo g, const uint8_t* 
   __syncthreads();
   at += base;
 #pragma unroll
-  for (int j = 0; j < kCells; ++j)
-    if (takes >> j & 1) list[at++] = (int)cell_of(n, j);
+  for (int j = 0; j < 4; ++j)
+    if (takes >> 8 * j & 1u) list[at++] = (int)(q.i + j);
 }
 
 // ---- the band pass (updateActiveFront and helpers, …extrapolation.wgsl.ts:172-331) ----
@@ -703,10 +764,15 @@ static void level_dims(int nx, int ny, int nz, std::vector<std::array<int, 3>>* 
   }
 }
 
+// Bytes on either side of a byte array that a quad's neighbour words reach
+// into (one plane and a word), aligned as the array is.
+static size_t quad_pad(int ny, int nz) { return ((size_t)ny * nz + 8 + 255) & ~(size_t)255; }
+
 size_t Extrapolator::estimate_bytes(int nx, int ny, int nz) {
   auto round = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t n = (size_t)nx * ny * nz;
-  size_t total = 2 * 6 * round(n * 4) + 4 * round(n) + round(n) + 2 * round(n) + round(n * 4) +
+  const size_t padded = n + 2 * quad_pad(ny, nz);
+  size_t total = 2 * 6 * round(n * 4) + 4 * round(n) + 3 * round(padded) + round(n * 4) +
                  round(sizeof(ExCounters)) + round(sizeof(ExTotals));
   total += round(n * 4) + round(((size_t)(nx + 1) * ny * nz + (size_t)nx * (ny + 1) * nz + (size_t)nx * ny * (nz + 1)) * 4);
   std::vector<std::array<int, 3>> dims;
@@ -734,9 +800,11 @@ int Extrapolator::create(int nx, int ny, int nz, double h) {
     if ((rc = alloc((void**)&st_[k].flags, n))) return rc;
     if ((rc = alloc((void**)&st_[k].stat, n))) return rc;
   }
-  if ((rc = alloc((void**)&cls_, n))) return rc;
-  if ((rc = alloc((void**)&cand_[0], n))) return rc;
-  if ((rc = alloc((void**)&cand_[1], n))) return rc;
+  const size_t pad = quad_pad(ny, nz);
+  for (uint8_t** p : {&cls_, &cand_[0], &cand_[1]}) {
+    if ((rc = alloc((void**)p, n + 2 * pad))) return rc;
+    *p += pad;
+  }
   if ((rc = alloc((void**)&list_, n * 4))) return rc;
   if ((rc = alloc((void**)&counters_, sizeof(ExCounters)))) return rc;
   if ((rc = alloc((void**)&totals_, sizeof(ExTotals)))) return rc;

@@ -62,7 +62,7 @@ class Extrapolator {
   // One extrapolation of a->phi / a->density and a->u, a->v, a->w into the
   // outputs; synchronous on s.
   // same_band: the field (phi / density) and open_top are those of this
-  // object's previous run, whose classes, near mask and band list are reused
+  // object's previous run, whose classes, list mask and band list are reused
   // (a second extrapolation over the same surface, as a MacCormack step makes)
   int run(hipStream_t s, const fp_extrapolate_args* a, fp_extrapolate_report* rep, bool same_band = false);
   size_t bytes() const { return bytes_; }

@@ -653,8 +653,134 @@ __global__ __launch_bounds__(kThreads) void k_ex_restrict(ExSrc src, ExLevel tgt
   tgt.known[i] = (uint8_t)known;
 }
 
-// prolongUnknownVelocity (…wgsl.ts:473-488) into a level's up arrays
-__global__ __launch_bounds__(kThreads) void k_ex_prolong(ExSrc src, ExLevel tgt, FastDiv tz, FastDiv ty) {
+// ---- prolongation of a tile ----
+// The target level in tiles of kTileX x kTileY x kTileZ cells, a lane per
+// (y, z) column.  hier_sample reads eight corners per component from the
+// coarser level, and neighbouring cells read the same ones: 48 gathers a cell,
+// and nine divisions for the sample positions, bound the prolongations.  Here
+// the coarse cells under the tile are staged in LDS once, per component as
+// (value or 0, known 1 or 0), with the coarse index clamped at staging; a
+// lane's y and z positions are made once for its kTileX cells.  A sample is
+// then eight LDS reads at fixed offsets and the sums of hier_sample, in its
+// order.
+constexpr int kTileX = 4, kTileY = 8, kTileZ = 32;
+// coarse cells under a tile: about half its extent, the far corner, the one
+// cell between the centred and the face sample, and one for odd levels' ratio
+constexpr int kWinX = 6, kWinY = 8, kWinZ = 20, kWin = kWinX * kWinY * kWinZ;
+
+struct TilePos {  // one axis of a sample: window index of the lower corner, fraction
+  int lo;
+  float fr;
+};
+__device__ __forceinline__ float sample_pos(int p, int S, int T, bool face) {
+  return face ? (float)(p + 1) * (float)S / (float)T - 1.0f : ((float)p + 0.5f) * (float)S / (float)T - 0.5f;
+}
+__device__ __forceinline__ TilePos tile_pos(int p, int S, int T, bool face, int base) {
+  const float pos = sample_pos(p, S, T, face), f = floorf(pos);
+  return TilePos{(int)f - base, pos - f};
+}
+// First coarse cell under target cells p0 .. p1 of an axis and their number
+__device__ __forceinline__ void tile_window(int p0, int p1, int S, int T, int& base, int& count) {
+  base = (int)floorf(fminf(sample_pos(p0, S, T, false), sample_pos(p0, S, T, true)));
+  count = (int)floorf(fmaxf(sample_pos(p1, S, T, false), sample_pos(p1, S, T, true))) + 2 - base;
+}
+
+// The sample of component c (hier_sample's corners and sums)
+__device__ __forceinline__ float tile_sample(const float2* win, const TilePos* ax, float* value) {
+  const float2* w = win + (ax[0].lo * kWinY + ax[1].lo) * kWinZ + ax[2].lo;
+  float cx[8], cw[8];
+#pragma unroll
+  for (int corner = 0; corner < 8; ++corner) {
+    const int o0 = corner & 1, o1 = corner >> 1 & 1, o2 = corner >> 2 & 1;
+    const float weight = (o0 ? ax[0].fr : 1.0f - ax[0].fr) * (o1 ? ax[1].fr : 1.0f - ax[1].fr) *
+                         (o2 ? ax[2].fr : 1.0f - ax[2].fr);
+    const float2 v = w[(o0 * kWinY + o1) * kWinZ + o2];
+    cx[corner] = weight > 0.0f ? weight * v.x : 0.0f;  // (a corner without weight may hold an infinity)
+    cw[corner] = weight * v.y;
+  }
+  const float xs = ((cx[0] + cx[5]) + (cx[1] + cx[4])) + ((cx[2] + cx[7]) + (cx[3] + cx[6]));
+  const float wsum = ((cw[0] + cw[5]) + (cw[1] + cw[4])) + ((cw[2] + cw[7]) + (cw[3] + cw[6]));
+  *value = wsum > 0.0f ? xs / wsum : 0.0f;
+  return wsum;
+}
+
+// Samples the unknown components of a lane's kTileX cells: known bits and
+// values (c, cell) in and out.  need: some lane of the workgroup has one (the
+// whole workgroup calls this with the same).  T: the target level.
+__device__ __forceinline__ void tile_fill(const ExSrc& S, const int* T, int x0, int y0, int z0, float2* win,
+                                          unsigned (&known)[kTileX], float (&val)[kTileX][3]) {
+  int base[3], m[3];
+  const int p0[3] = {x0, y0, z0};
+  const int tile[3] = {kTileX, kTileY, kTileZ};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) tile_window(p0[a], min(p0[a] + tile[a], T[a]) - 1, S.d[a], T[a], base[a], m[a]);
+  const int tid = (int)threadIdx.x;
+  const int y = y0 + (tid / kTileZ), z = z0 + tid % kTileZ;
+  if (m[0] > kWinX || m[1] > kWinY || m[2] > kWinZ) {  // no level ratio makes such a window; sampled directly
+    for (int j = 0; j < kTileX; ++j) {
+      const int p[3] = {x0 + j, y, z};
+      if (p[0] >= T[0] || y >= T[1] || z >= T[2]) continue;
+      for (int c = 0; c < 3; ++c) {
+        float v;
+        if (!(known[j] >> c & 1) && hier_sample(S, T, p, c, &v) > 0.0f) {
+          val[j][c] = v;
+          known[j] |= 1u << c;
+        }
+      }
+    }
+    return;
+  }
+  for (int q = tid; q < m[0] * m[1] * m[2]; q += kThreads) {
+    const int d = q % m[2], t = q / m[2], b = t % m[1], a = t / m[1];
+    const int X = min(max(base[0] + a, 0), S.d[0] - 1), Y = min(max(base[1] + b, 0), S.d[1] - 1),
+              Z = min(max(base[2] + d, 0), S.d[2] - 1);
+    const unsigned i = ((unsigned)X * S.d[1] + Y) * S.d[2] + Z;
+    const unsigned kn = S.known[i];
+    const float v[3] = {S.val[0][i], S.val[1][i], S.val[2][i]};
+    const int o = (a * kWinY + b) * kWinZ + d;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const bool k = kn >> c & 1;
+      win[c * kWin + o] = make_float2(k ? v[c] : 0.0f, k ? 1.0f : 0.0f);
+    }
+  }
+  __syncthreads();
+  if (y >= T[1] || z >= T[2]) return;
+  const TilePos py[2] = {tile_pos(y, S.d[1], T[1], false, base[1]), tile_pos(y, S.d[1], T[1], true, base[1])};
+  const TilePos pz[2] = {tile_pos(z, S.d[2], T[2], false, base[2]), tile_pos(z, S.d[2], T[2], true, base[2])};
+#pragma unroll
+  for (int j = 0; j < kTileX; ++j) {
+    if (x0 + j >= T[0] || known[j] == 7u) continue;
+    const TilePos px[2] = {tile_pos(x0 + j, S.d[0], T[0], false, base[0]),
+                           tile_pos(x0 + j, S.d[0], T[0], true, base[0])};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (known[j] >> c & 1) continue;
+      const TilePos ax[3] = {px[c == 0], py[c == 1], pz[c == 2]};
+      float v;
+      if (tile_sample(win + c * kWin, ax, &v) > 0.0f) {
+        val[j][c] = v;
+        known[j] |= 1u << c;
+      }
+    }
+  }
+}
+
+// tile of a launch over the level's tiles (z fastest), in XCD-contiguous runs
+__device__ __forceinline__ bool tile_of(const int* T, int& x0, int& y0, int& z0) {
+  const unsigned tz = (T[2] + kTileZ - 1) / kTileZ, ty = (T[1] + kTileY - 1) / kTileY, tx = (T[0] + kTileX - 1) / kTileX;
+  const unsigned t = chunk_of(tx * ty * tz);
+  if (t >= tx * ty * tz) return false;
+  z0 = (int)(t % tz) * kTileZ;
+  y0 = (int)(t / tz % ty) * kTileY;
+  x0 = (int)(t / (tz * ty)) * kTileX;
+  return true;
+}
+
+// prolongUnknownVelocity (…wgsl.ts:473-488) into a level's up arrays, a lane
+// per cell: for levels too small to fill the chip with tiles, where a tile's
+// staging is one more round trip (0.34 M cells: 11.6 us, 15.9 in tiles)
+__global__ __launch_bounds__(kThreads) void k_ex_prolong_cells(ExSrc src, ExLevel tgt, FastDiv tz, FastDiv ty) {
   const unsigned n = (unsigned)tgt.n;
   const unsigned i = chunk_of((n + kThreads - 1) / kThreads) * kThreads + threadIdx.x;
   if (i >= n) return;
@@ -674,51 +800,86 @@ __global__ __launch_bounds__(kThreads) void k_ex_prolong(ExSrc src, ExLevel tgt,
   }
   tgt.up_known[i] = (uint8_t)known;
 }
+constexpr long long kTileCells = 1 << 20;  // levels of this many cells take tiles
+
+// The same in tiles: 113 us -> 74 on the 192^3 level.
+__global__ __launch_bounds__(kThreads) void k_ex_prolong(ExSrc src, ExLevel tgt) {
+  __shared__ float2 win[3 * kWin];
+  int x0, y0, z0;
+  if (!tile_of(tgt.d, x0, y0, z0)) return;
+  const int y = y0 + (int)threadIdx.x / kTileZ, z = z0 + (int)threadIdx.x % kTileZ;
+  const bool column = y < tgt.d[1] && z < tgt.d[2];
+  unsigned known[kTileX];
+  float val[kTileX][3];
+  bool need = false;
+#pragma unroll
+  for (int j = 0; j < kTileX; ++j) {
+    const bool in = column && x0 + j < tgt.d[0];
+    const unsigned i = in ? ((unsigned)(x0 + j) * tgt.d[1] + y) * tgt.d[2] + z : 0u;
+    known[j] = in ? tgt.known[i] : 7u;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) val[j][c] = tgt.val[c][i];
+    need = need || known[j] != 7u;
+  }
+  if (__syncthreads_or(need)) tile_fill(src, tgt.d, x0, y0, z0, win, known, val);
+#pragma unroll
+  for (int j = 0; j < kTileX; ++j) {
+    if (!column || x0 + j >= tgt.d[0]) continue;
+    const unsigned i = ((unsigned)(x0 + j) * tgt.d[1] + y) * tgt.d[2] + z;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) tgt.up_val[c][i] = val[j][c];
+    tgt.up_known[i] = (uint8_t)known[j];
+  }
+}
 
 // the last prolongation onto the band result, packed into the face arrays
-// (packTransportShell, …wgsl.ts:491-512): known values on open faces, 0 else
+// (packTransportShell, …wgsl.ts:491-512): known values on open faces, 0 else.
+// 990 us at 384^3 with a lane per cell, 654 in tiles, 39.7 against 52 at
+// 160 x 117 x 143; 24 bytes a cell at most, 2.1 TB/s: what is left is the sums.
 __global__ __launch_bounds__(kThreads) void k_ex_finish(ExGeo g, ExSrc src, int have_src, ExState r,
                                                        const uint8_t* __restrict__ cls, ExCounters* cnt,
                                                        float* __restrict__ uo, float* __restrict__ vo,
-                                                       float* __restrict__ wo, unsigned n) {
+                                                       float* __restrict__ wo) {
+  __shared__ float2 win[3 * kWin];
+  int x0 = 0, y0 = 0, z0 = 0;
+  if (!tile_of(g.d, x0, y0, z0)) return;
+  const int y = y0 + (int)threadIdx.x / kTileZ, z = z0 + (int)threadIdx.x % kTileZ;
+  const bool column = y < g.d[1] && z < g.d[2];
   int unknown = 0, band = 0;
-  unsigned mes[kCells], knowns[kCells];
-  float owns[kCells][3];
+  unsigned me[kTileX], known[kTileX];
+  float val[kTileX][3];
+  bool need = false;
 #pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = min(cell_of(n, j), n - 1);
-    mes[j] = cls[i];
-    knowns[j] = r.flags[i] & 7u;
-    owns[j][0] = r.val[0][i];
-    owns[j][1] = r.val[1][i];
-    owns[j][2] = r.val[2][i];
+  for (int j = 0; j < kTileX; ++j) {
+    const bool in = column && x0 + j < g.d[0];
+    const unsigned i = in ? eidx(g, x0 + j, y, z) : 0u;
+    me[j] = in ? cls[i] : 0u;
+    known[j] = in ? r.flags[i] & 7u : 0u;
   }
+  // (the band result holds no values in the far air, most of a tank)
 #pragma unroll
-  for (int j = 0; j < kCells; ++j) {
-    const unsigned i = cell_of(n, j);
-    if (i >= n) break;
-    int x, y, z;
-    edecode(g, i, x, y, z);
-    const unsigned me = mes[j];
-    const unsigned known = knowns[j];
-    const float* own = owns[j];
-    band += __popc(known);
-    const int p[3] = {x, y, z};
+  for (int j = 0; j < kTileX; ++j) {
+    const unsigned i = column && x0 + j < g.d[0] ? eidx(g, x0 + j, y, z) : 0u;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) val[j][c] = 0.0f;
+    if (known[j])
+#pragma unroll
+      for (int c = 0; c < 3; ++c) val[j][c] = r.val[c][i];
+    band += __popc(known[j]);
+    // a closed face is written 0 whatever the hierarchy holds
+    known[j] |= ~me[j] & 7u;
+    need = need || known[j] != 7u;
+  }
+  if (__syncthreads_or(need) && have_src) tile_fill(src, g.d, x0, y0, z0, win, known, val);
+#pragma unroll
+  for (int j = 0; j < kTileX; ++j) {
+    const int x = x0 + j;
+    if (!column || x >= g.d[0]) continue;
+    const unsigned open = me[j] & 7u;
+    unknown += __popc(open & ~known[j]);
     float* out[3] = {uo, vo, wo};
-    for (int c = 0; c < 3; ++c) {
-      float val = own[c];
-      bool k = known >> c & 1;
-      if (!k && have_src) {
-        float v;
-        if (hier_sample(src, g.d, p, c, &v) > 0.0f) {
-          val = v;
-          k = true;
-        }
-      }
-      const bool open = me >> c & 1;
-      if (open && !k) unknown += 1;
-      out[c][face_of(g, c, x, y, z)] = open && k ? val : 0.0f;
-    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out[c][face_of(g, c, x, y, z)] = (open & known[j]) >> c & 1u ? val[j][c] : 0.0f;
     // the negative domain faces are walls
     if (x == 0) uo[(unsigned)y * g.d[2] + z] = 0.0f;
     if (y == 0) vo[(unsigned)x * (g.d[1] + 1) * g.d[2] + z] = 0.0f;
@@ -731,6 +892,13 @@ __global__ __launch_bounds__(kThreads) void k_ex_finish(ExGeo g, ExSrc src, int 
     if (su) atomicAdd(&cnt->unknown[blockIdx.x % kExSpread][0], (unsigned long long)su);
     if (sb) atomicAdd(&cnt->band_known[blockIdx.x % kExSpread][0], (unsigned long long)sb);
   }
+}
+
+// workgroups of a launch over a level's tiles
+int tiled_grid(const int* d) {
+  auto up = [](int n, int t) { return (n + t - 1) / t; };
+  const int tiles = up(d[0], kTileX) * up(d[1], kTileY) * up(d[2], kTileZ);
+  return 8 * ((tiles + 7) / 8);
 }
 
 // workgroups of a streaming launch over n < 2^31 items, cells per thread k
@@ -928,12 +1096,15 @@ int Extrapolator::run(hipStream_t s, const fp_extrapolate_args* a, fp_extrapolat
   }
   for (int l = L - 2; l >= 0; --l) {
     const ExLevel& T = levels_[l];
-    hipLaunchKernelGGL(k_ex_prolong, dim3(chunked_grid(T.n)), block, 0, s, coarser, T, make_div((unsigned)T.d[2]),
-                       make_div((unsigned)T.d[1]));
+    if (T.n >= kTileCells)
+      hipLaunchKernelGGL(k_ex_prolong, dim3(tiled_grid(T.d)), block, 0, s, coarser, T);
+    else
+      hipLaunchKernelGGL(k_ex_prolong_cells, dim3(chunked_grid(T.n)), block, 0, s, coarser, T,
+                         make_div((unsigned)T.d[2]), make_div((unsigned)T.d[1]));
     coarser = ExSrc{{T.d[0], T.d[1], T.d[2]}, {T.up_val[0], T.up_val[1], T.up_val[2]}, T.up_known};
   }
-  hipLaunchKernelGGL(k_ex_finish, grid, block, 0, s, g, coarser, L > 0 ? 1 : 0, st_[0], (const uint8_t*)cls_,
-                     counters_, uo, vo, wo, un);
+  hipLaunchKernelGGL(k_ex_finish, dim3(tiled_grid(d_)), block, 0, s, g, coarser, L > 0 ? 1 : 0, st_[0],
+                     (const uint8_t*)cls_, counters_, uo, vo, wo);
   if (a->memory == FP_MEMORY_HOST) {
     HIPCHK(hipMemcpyAsync(a->u_out, uo, nu * 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(a->v_out, vo, nv * 4, hipMemcpyDeviceToHost, s));

@@ -37,10 +37,11 @@ class Advector {
   int d_[3] = {0, 0, 0};
   float h_ = 0.0f;
   size_t nf_[3] = {0, 0, 0};
-  float* transport_ = nullptr;  // the current field's extrapolation, when the caller gives none
+  float* transport_ = nullptr;  // the current field's extrapolation, when the caller gives none; then
+                                // the MacCormack prediction's
   float* pred_ = nullptr;       // MacCormack prediction
-  float* rev_ = nullptr;        // MacCormack reverse advection
-  float* pred_ext_ = nullptr;   // the prediction's extrapolation
+  float* lower_ = nullptr;      // range of its donors
+  float* upper_ = nullptr;
   float* out_ = nullptr;        // output staging (host memory or outputs overlapping inputs)
   float* host_ = nullptr;       // input staging for host memory
   size_t host_floats_ = 0;

@@ -1,0 +1,35 @@
+"""The advection's sample paths on the GPU: cells at every wall and edge of
+grids down to two cells, rows that end inside a wave, flows of a fraction of a
+cell and of several pieces, no flow, tiny and huge values, and quotients by h
+either side of where the division takes over.  Bar: bit for bit against
+the CPU restatement, both schemes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (2, 5, 66), (3, 2, 130), (17, 9, 2), (12, 20, 64), (21, 18, 33)])
+@pytest.mark.parametrize("scheme", ["semi-lagrangian", "maccormack"])
+def test_paths_bit_exact(fpl, oracle, dims, scheme):
+    rng = np.random.default_rng(sum(dims))
+    h = 1.0 / max(dims)
+    y = np.arange(dims[1]) + 0.5
+    phi = np.broadcast_to((y - 0.6 * dims[1])[None, :, None] * h, dims).astype(np.float32).copy()
+    shapes = [(dims[0] + (a == 0), dims[1] + (a == 1), dims[2] + (a == 2)) for a in range(3)]
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        for cells, top in ((0.3, False), (0.3, True), (2.7, False), (9.0, True), (0.0, False), (1e-30, True),
+                           (1e30, False), (None, True)):
+            dt = 0.01
+            field = [(rng.standard_normal(s) * cells * h / dt if cells is not None else
+                      rng.uniform(-1.2e38, 1.2e38, s) * h).astype(np.float32) for s in shapes]
+            cur = [(rng.standard_normal(s)).astype(np.float32) for s in shapes]
+            want = oracle.advect_velocity(*cur, h, dt, phi=phi, transport=field, gravity=-9.81, nu=1e-3, scheme=scheme,
+                                          open_top=int(top))
+            got = g.advect(*cur, dt, phi=phi, transport=field, gravity=-9.81, viscosity=1e-3, scheme=scheme,
+                           open_top=top)
+            for a, b in zip(got[:3], want):
+                assert np.array_equal(a, b, equal_nan=True), (cells, top)
+    finally:
+        g.destroy()

@@ -62,7 +62,7 @@ struct TallRec {
   const int* bases;    // (nx, nz)
   float* phi;          // samples (private copy)
   TallCol* cols;       // (nx, nz)
-  int* top;            // (nx, nz): highest packed band row holding liquid (1: none)
+  int* top;            // (nx, nz): class word (class_top, class_deep, class_pair)
   fp_f32x4* blk;       // per column: inverse (bottom, top) block bb, bt, tt and 0
   float* dinv;         // per sample: inverse diagonal of band unknowns
   double* b;           // FP64 right-hand side

@@ -1,0 +1,53 @@
+"""Band segments of tall-cell columns, in liquid and at the surface, against the
+FP64 oracle: bands that are no multiple of a segment, columns that end inside a
+wave or start a second one, a smooth deep tank whose waves hold liquid alone, a
+rough one where they mix, tall samples of a tiny negative level, infinite
+levels in the air, and a band that reaches the lid.
+
+Bars: the operator's refinement reaches 1e-10 and the pressure the oracle's to
+1e-7.  A pass of the inner solve ends at a residual 1e-4 of its start or less
+and FP32 operators that agree with the FP64 one to a few ulp keep that gain, so
+six passes are enough."""
+import numpy as np
+import pytest
+
+from fluid_amd import scenes
+from fluid_amd import tall_layout as tl
+
+pytestmark = pytest.mark.gpu
+
+
+def tank(nx, nz, ny, band, depth, rough, slope, seed):
+    """Surface `depth` rows above the bases, which vary by at most `slope`."""
+    rng = np.random.default_rng(seed)
+    h = 1.0 / ny
+    raw = np.full((nx, nz), ny - band - 1 if depth < band else ny - band, np.int32)
+    raw -= rng.integers(0, slope + 1, (nx, nz)).astype(np.int32)
+    L = tl.TallCellLayout(tl.limit_bases(np.maximum(raw, 2), 4), ny, band, h, 4)
+    surf = (np.asarray(L.bases, np.float64) + depth + rng.uniform(-rough, rough, (nx, nz))) * h
+    phi = np.clip(L.sample_heights() * h - surf[:, None, :], -5 * h, 5 * h)
+    return L, np.where(L.active(), phi, 5 * h).astype(np.float32), rng
+
+
+@pytest.mark.parametrize("nx,nz,ny,band,depth,rough,slope,edit", [
+    (9, 70, 40, 13, 9.4, 0.3, 0, ""), (8, 64, 48, 16, 13.2, 0.2, 3, ""), (5, 257, 30, 10, 5.5, 3.0, 4, ""),
+    (16, 33, 60, 23, 18.6, 2.0, 2, "tiny"), (7, 40, 36, 12, 8.3, 1.0, 4, "infinite"), (6, 21, 24, 5, 9.0, 0.1, 1, ""),
+])
+def test_segments_match_oracle(fpl, oracle, nx, nz, ny, band, depth, rough, slope, edit):
+    L, phi, rng = tank(nx, nz, ny, band, depth, rough, slope, nx * nz)
+    if edit == "tiny":
+        phi[:, 1, ::3] = -1e-12
+    if edit == "infinite":
+        phi[phi > 0] = np.inf
+    masks = scenes.tall_fluid_slots(L, np.where(np.isinf(phi), np.float32(5 * L.h), phi))
+    u, v, w = (np.where(m, rng.standard_normal(m.shape) * 0.3, 0.0).astype(np.float32) for m in masks)
+    want = oracle.Tall(L.bases, phi, L.fine_ny, L.band, L.h, L.max_delta).projection(u, v, w, 0.01, 1000.0,
+                                                                                      rel_tol=1e-12)[0]
+    g = fpl.TallCellPressureProjection.from_layout(L)
+    try:
+        got = g.project(phi, u, v, w, 0.01, 1000.0, relative_tolerance=1e-10)
+        print(got.report["iterations"], got.report["outer_iterations"])
+        assert got.report["relative_residual"] <= 1e-10 and got.report["outer_iterations"] <= 6
+        assert np.linalg.norm(got.pressure - want) <= 1e-7 * np.linalg.norm(want)
+    finally:
+        g.destroy()

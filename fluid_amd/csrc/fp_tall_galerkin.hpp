@@ -458,18 +458,32 @@ __device__ __forceinline__ void lat_prolong_node(const TallRec& G, int level, in
   ef[i] += ec[((size_t)(x >> 1) * C.ny + coarse_row(y, C.cy)) * C.nz + (z >> 1)];
 }
 
+// Nodes i of a level, FP_BLOCK to a turn: with a stride that divides by 8 the
+// turns are dealt to the XCDs (workgroup b runs on XCD b % 8) in eight runs of
+// consecutive nodes, so that the couplings and values a node reads from its -x
+// neighbour's slab were just read on the same XCD and are in its L2 (dealt one
+// by one they came from memory: 189 MB a sweep of level 1 of 512^2 columns,
+// whose couplings and vectors are 128 MB).  A sweep there 41 -> 37 us, the
+// levels' mean 12.0 -> 10.3.
+#define LAT_NODES(i, n)                                                                                    \
+  for (unsigned turns_ = (unsigned)(((n) + FP_BLOCK - 1) / FP_BLOCK), xcds_ = (nblk & 7) == 0 ? 8u : 1u,   \
+                run_ = (turns_ + xcds_ - 1) / xcds_, first_ = (unsigned)blk % xcds_ * run_,                \
+                turn_ = first_ + (unsigned)blk / xcds_;                                                    \
+       turn_ < min(first_ + run_, turns_); turn_ += (unsigned)nblk / xcds_)                                \
+    if (const size_t i = (size_t)turn_ * FP_BLOCK + threadIdx.x; i < (n))
+
 __global__ void k_lat_jacobi(const TallPart* parts, int np, int level, int sel, int first) {
   FP_PART(parts, np);
   if (G.st->done) return;
   const int kh = cload(G.reach + 2 * level), kv = cload(G.reach + 2 * level + 1);
-  FP_STRIDE(i, (size_t)G.lv[level].n) lat_jacobi_node(G, level, sel, first, kh, kv, i);
+  LAT_NODES(i, (size_t)G.lv[level].n) lat_jacobi_node(G, level, sel, first, kh, kv, i);
 }
 
 __global__ void k_lat_residual(const TallPart* parts, int np, int level, int sel) {
   FP_PART(parts, np);
   if (G.st->done) return;
   const int kh = cload(G.reach + 2 * level), kv = cload(G.reach + 2 * level + 1);
-  FP_STRIDE(i, (size_t)G.lv[level].n) lat_residual_node(G, level, sel, kh, kv, i);
+  LAT_NODES(i, (size_t)G.lv[level].n) lat_residual_node(G, level, sel, kh, kv, i);
 }
 
 __global__ void k_lat_restrict(const TallPart* parts, int np, int level) {
@@ -481,7 +495,7 @@ __global__ void k_lat_restrict(const TallPart* parts, int np, int level) {
 __global__ void k_lat_prolong(const TallPart* parts, int np, int level, int sel) {
   FP_PART(parts, np);
   if (G.st->done) return;
-  FP_STRIDE(i, (size_t)G.lv[level].n) lat_prolong_node(G, level, sel, i);
+  LAT_NODES(i, (size_t)G.lv[level].n) lat_prolong_node(G, level, sel, i);
 }
 
 // Dense FP64 inverse of the coarsest lattice (one workgroup per grid).  As on

@@ -212,42 +212,58 @@ __global__ __launch_bounds__(FP_BLOCK) void k_tall_galerkin1(const TallPart* par
 // Every coupling of a level-l node i, emitted as (neighbour X, Y, Z, a).
 // kh / kv bound the row offsets visited for the x/z and the same-column
 // couplings (K, K visit the whole band; a level's measured reach skips slots
-// that are zero on every node).
+// that are zero on every node).  The couplings are loaded kEntryRows row
+// offsets at a time, clamped to the node itself where a neighbour is missing,
+// and only then tested and emitted: a test behind each load made a chain of 45
+// round trips a node (k_tall_galerkin of 512^2 columns' lattice levels, the mean
+// of six: 90 -> 63 us).
+constexpr int kEntryRows = 3;
 template <class Emit>
 __device__ void lattice_row_entries(const TallLevel& L, int K, int kh, int kv, int x, int y, int z, Emit& emit) {
   const size_t n = (size_t)L.n;
   const float* __restrict__ w = L.w;
-  auto at = [&](int xx, int yy, int zz) { return ((size_t)xx * L.ny + yy) * L.nz + zz; };
-  const size_t i = at(x, y, z);
+  const size_t sy = (size_t)L.nz, sx = (size_t)L.ny * L.nz;
+  const size_t i = (size_t)x * sx + (size_t)y * sy + z;
+  const bool xp = x + 1 < L.nx, xm = x > 0, zp = z + 1 < L.nz, zm = z > 0;
   emit(x, y, z, w[(size_t)slot_d(K) * n + i]);
-  for (int dy = -kh; dy <= kh; ++dy) {
-    const int yy = y + dy;
-    if (yy < 0 || yy >= L.ny) continue;
-    if (x + 1 < L.nx) {
-      const float v = w[(size_t)slot_x(K, dy) * n + i];
-      if (v != 0.0f) emit(x + 1, yy, z, v);
+  for (int dy0 = -kh; dy0 <= kh; dy0 += kEntryRows) {
+    float v[kEntryRows][4];
+#pragma unroll
+    for (int r = 0; r < kEntryRows; ++r) {
+      const int dy = min(dy0 + r, kh), yy = y + dy;
+      const bool row = yy >= 0 && yy < L.ny;
+      const size_t j = i + (size_t)((long long)(row ? dy : 0) * (long long)sy);  // (x, yy, z), clamped
+      v[r][0] = w[(size_t)slot_x(K, dy) * n + i];
+      // stored by (x-1, yy) towards (x, y): offset -dy
+      v[r][1] = w[(size_t)slot_x(K, -dy) * n + (xm ? j - sx : j)];
+      v[r][2] = w[(size_t)slot_z(K, dy) * n + i];
+      v[r][3] = w[(size_t)slot_z(K, -dy) * n + (zm ? j - 1 : j)];
     }
-    if (x > 0) {  // stored by (x-1, yy) towards (x, y): offset -dy
-      const float v = w[(size_t)slot_x(K, -dy) * n + at(x - 1, yy, z)];
-      if (v != 0.0f) emit(x - 1, yy, z, v);
-    }
-    if (z + 1 < L.nz) {
-      const float v = w[(size_t)slot_z(K, dy) * n + i];
-      if (v != 0.0f) emit(x, yy, z + 1, v);
-    }
-    if (z > 0) {
-      const float v = w[(size_t)slot_z(K, -dy) * n + at(x, yy, z - 1)];
-      if (v != 0.0f) emit(x, yy, z - 1, v);
+#pragma unroll
+    for (int r = 0; r < kEntryRows; ++r) {
+      const int yy = y + dy0 + r;
+      if (dy0 + r > kh || yy < 0 || yy >= L.ny) continue;
+      if (xp && v[r][0] != 0.0f) emit(x + 1, yy, z, v[r][0]);
+      if (xm && v[r][1] != 0.0f) emit(x - 1, yy, z, v[r][1]);
+      if (zp && v[r][2] != 0.0f) emit(x, yy, z + 1, v[r][2]);
+      if (zm && v[r][3] != 0.0f) emit(x, yy, z - 1, v[r][3]);
     }
   }
-  for (int dy = 1; dy <= kv; ++dy) {
-    if (y + dy < L.ny) {
-      const float v = w[(size_t)slot_y(K, dy) * n + i];
-      if (v != 0.0f) emit(x, y + dy, z, v);
+  for (int dy0 = 1; dy0 <= kv; dy0 += kEntryRows) {
+    float v[kEntryRows][2];
+#pragma unroll
+    for (int r = 0; r < kEntryRows; ++r) {
+      const int dy = min(dy0 + r, kv);
+      const float* __restrict__ ws = w + (size_t)slot_y(K, dy) * n + i;
+      v[r][0] = ws[0];
+      v[r][1] = *(y - dy >= 0 ? ws - (size_t)dy * sy : ws);
     }
-    if (y - dy >= 0) {
-      const float v = w[(size_t)slot_y(K, dy) * n + at(x, y - dy, z)];
-      if (v != 0.0f) emit(x, y - dy, z, v);
+#pragma unroll
+    for (int r = 0; r < kEntryRows; ++r) {
+      const int dy = dy0 + r;
+      if (dy > kv) continue;
+      if (y + dy < L.ny && v[r][0] != 0.0f) emit(x, y + dy, z, v[r][0]);
+      if (y - dy >= 0 && v[r][1] != 0.0f) emit(x, y - dy, z, v[r][1]);
     }
   }
 }
@@ -320,9 +336,12 @@ __global__ void k_tall_l1diag(const TallPart* parts, int np, int level) {
     kh = max(kh, __shfl_xor(kh, o, 64));
     kv = max(kv, __shfl_xor(kv, o, 64));
   }
+  // (a wave that knows of a larger one leaves the counter alone: the atomics of
+  // 16 thousand waves on one address took 0.36 ms)
   if ((threadIdx.x & 63) == 0) {
-    atomicMax(G.reach + 2 * level, kh);
-    atomicMax(G.reach + 2 * level + 1, kv);
+    int* reach = G.reach + 2 * level;
+    if (kh > __hip_atomic_load(reach, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(reach, kh);
+    if (kv > __hip_atomic_load(reach + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(reach + 1, kv);
   }
 }
 
@@ -498,7 +517,10 @@ __global__ void k_lat_prolong(const TallPart* parts, int np, int level, int sel)
   LAT_NODES(i, (size_t)G.lv[level].n) lat_prolong_node(G, level, sel, i);
 }
 
-// Dense FP64 inverse of the coarsest lattice (one workgroup per grid).  As on
+// Dense FP64 inverse of the coarsest lattice (one workgroup per grid, the matrix
+// in LDS: its m steps are m chains of three barriers; m = 27: 123 -> 35 us,
+// m = 48: 286 -> 99 us, where the matrix and the search of each coupling's row
+// were in memory).  As on
 // uniform grids, the vanishing last pivot of a component without an air face
 // (a grid that is liquid everywhere, its band up to the lid) gets its row's
 // original diagonal added: the inverse of A + a_pp e_p e_p^T, SPD.
@@ -506,18 +528,22 @@ __global__ void k_tall_coarse_setup(const TallPart* parts) {
   const TallRec& G = *parts[blockIdx.x].g;
   const TallLevel& L = G.lv[G.L - 1];
   const int K = G.K;
-  int* __restrict__ cmap = G.cmap;
-  double* __restrict__ a = G.minv;
+  __shared__ double a[kTallMaxCoarse * kTallMaxCoarse];
+  __shared__ int cmap[kTallMaxCoarse], s_row[kTallMaxCoarse];  // node of a row, row of a node (-1: inactive)
   __shared__ int s_n, s_fail;
   __shared__ double s_diag[kTallMaxCoarse];
-  const size_t n = (size_t)L.n;
-  if (threadIdx.x == 0) {
-    int c = 0;
-    for (size_t i = 0; i < n && c < G.max_coarse; ++i)
-      if (L.w[(size_t)slot_d(K) * n + i] > 0.0f) cmap[c++] = (int)i;
-    s_n = c;
-    s_fail = 0;
-    *G.ncoarse = c;
+  const size_t n = (size_t)L.n;  // at most kTallMaxCoarse: the plan ends there
+  if (threadIdx.x < 64) {
+    const bool active = threadIdx.x < n && L.w[(size_t)slot_d(K) * n + threadIdx.x] > 0.0f;
+    const unsigned long long all = __ballot(active);
+    const int c = __popcll(all & ((1ull << threadIdx.x) - 1));
+    s_row[threadIdx.x] = active ? c : -1;
+    if (active) G.cmap[c] = cmap[c] = (int)threadIdx.x;
+    if (threadIdx.x == 0) {
+      s_n = __popcll(all);
+      s_fail = 0;
+      *G.ncoarse = s_n;
+    }
   }
   __syncthreads();
   const int m = s_n;
@@ -531,12 +557,8 @@ __global__ void k_tall_coarse_setup(const TallPart* parts) {
     const int y = (int)(tt % (size_t)L.ny);
     const int x = (int)(tt / (size_t)L.ny);
     auto emit = [&](int xj, int yj, int zj, float v) {
-      const size_t j = ((size_t)xj * L.ny + yj) * L.nz + zj;
-      for (int c = 0; c < m; ++c)
-        if ((size_t)cmap[c] == j) {
-          a[(size_t)r * m + c] += (double)v;
-          break;
-        }
+      const int c = s_row[((size_t)xj * L.ny + yj) * L.nz + zj];
+      if (c >= 0) a[r * m + c] += (double)v;
     };
     lattice_row_entries(L, K, K, K, x, y, z, emit);
   }
@@ -571,7 +593,9 @@ __global__ void k_tall_coarse_setup(const TallPart* parts) {
     for (int r = threadIdx.x; r < m; r += blockDim.x)
       a[r * m + r] = 1.0 / (double)L.w[(size_t)slot_d(K) * n + cmap[r]];
     if (threadIdx.x == 0) G.st->flags |= 0x40;  // FP_FLAG_COARSE_SINGULAR
+    __syncthreads();
   }
+  for (int e = threadIdx.x; e < m * m; e += blockDim.x) G.minv[e] = a[e];
 }
 
 // e = Minv r on the coarsest level's active nodes (the calling workgroup),

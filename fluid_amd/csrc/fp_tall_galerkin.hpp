@@ -616,10 +616,161 @@ __device__ __forceinline__ void coarse_solve_block(const TallRec& G) {
 // most kTallBottomNodes nodes each) are smoothed, restricted, solved on the
 // coarsest level and prolonged with the same steps and buffer conventions as
 // the grid kernels, separated by workgroup barriers instead of launches.
+static_assert(kTallBottomNodes <= kTallBottomThreads, "a thread per node");
+constexpr int kBottomReach = 3;  // the row offsets a node's registers hold
+
+// One node's couplings (zero where there is none) for |row offset| <= R.
+template <int R>
+struct NodeRow {
+  float d, xp[2 * R + 1], xm[2 * R + 1], zp[2 * R + 1], zm[2 * R + 1], yp[R], ym[R];
+  __device__ __forceinline__ void load(const TallLevel& L, int K, int kh, int kv, int i) {
+    int x, y, z;
+    node_xyz(L, (size_t)i, x, y, z);
+    const int n = (int)L.n, sy = L.nz, sx = L.ny * L.nz;
+    const float* __restrict__ w = L.w;
+    d = w[slot_d(K) * n + i];
+    const bool hp = x + 1 < L.nx, hm = x > 0, vp = z + 1 < L.nz, vm = z > 0;
+#pragma unroll
+    for (int r = 0; r < 2 * R + 1; ++r) {
+      const int dy = r - R, yy = y + dy;
+      const bool in = dy >= -kh && dy <= kh && yy >= 0 && yy < L.ny;
+      const int j = i + (in ? dy * sy : 0), o = in ? dy : 0;
+      xp[r] = in && hp ? w[slot_x(K, o) * n + i] : 0.0f;
+      xm[r] = in && hm ? w[slot_x(K, -o) * n + j - sx] : 0.0f;
+      zp[r] = in && vp ? w[slot_z(K, o) * n + i] : 0.0f;
+      zm[r] = in && vm ? w[slot_z(K, -o) * n + j - 1] : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int dy = r + 1;
+      yp[r] = dy <= kv && y + dy < L.ny ? w[slot_y(K, dy) * n + i] : 0.0f;
+      ym[r] = dy <= kv && y - dy >= 0 ? w[slot_y(K, dy) * n + i - dy * sy] : 0.0f;
+    }
+  }
+  // (A e)_i, e pointing at the node: lattice_apply's sums; a missing
+  // neighbour's place holds another node's value or the guard's zero
+  __device__ __forceinline__ float apply(const float* e, int sx, int sy) const {
+    float acc = d * e[0];
+#pragma unroll
+    for (int r = 0; r < 2 * R + 1; ++r) {
+      const float* ej = e + (r - R) * sy;
+      acc += (xp[r] * ej[sx] + xm[r] * ej[-sx]) + (zp[r] * ej[1] + zm[r] * ej[-1]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc += yp[r] * e[(r + 1) * sy] + ym[r] * e[-(r + 1) * sy];
+    return acc;
+  }
+};
+
+// Values of a level in LDS between zeros: a node's neighbours lie within nx-1
+// rows' slab and kBottomReach rows, less than kBottomGuard nodes away (a slab
+// has at most kTallBottomNodes nodes and, with its two tall rows and one band
+// row at least, three rows).
+constexpr int kBottomGuard = 2048;
+static_assert(kTallBottomNodes + kBottomReach * (kTallBottomNodes / 3) < kBottomGuard, "guards hold every neighbour");
+typedef float BottomValues[kBottomGuard + kTallBottomNodes + kBottomGuard];
+
+// The levels of one grid, a thread per node: its couplings in registers (each
+// sweep read them again from L2, a chain of some 18 such passes), the values in
+// LDS, the right-hand sides and the corrections before the coarse ones kept
+// by the thread that wrote them: 57 -> 23 us for 96^2 columns, 60 -> 27 us for
+// 512^2.
+template <int R>
+__device__ __forceinline__ void bottom_in_registers(const TallRec& G, BottomValues* vals) {
+  const int lb = G.lb, lc = G.L - 1, K = G.K, i = (int)threadIdx.x;
+  int at = 0;  // the buffer holding the level's correction
+  for (int l = lb; l < lc; ++l) {
+    const TallLevel& L = G.lv[l];
+    const TallLevel& C = G.lv[l + 1];
+    const int n = (int)L.n, sy = L.nz, sx = L.ny * L.nz;
+    NodeRow<R> row;
+    float di = 0.0f, r = 0.0f, e = 0.0f;
+    if (i < n) {
+      row.load(L, K, G.reach[2 * l], G.reach[2 * l + 1], i);
+      di = L.dinv[i];
+      r = L.r[i];
+      e = di != 0.0f ? r * di : 0.0f;
+      vals[at][kBottomGuard + i] = e;
+    }
+    __syncthreads();
+    for (int sw = 1; sw < kTallCoarseSweeps; ++sw, at ^= 1) {
+      if (i < n) {
+        e = di != 0.0f ? e + (r - row.apply(&vals[at][kBottomGuard + i], sx, sy)) * di : 0.0f;
+        vals[at ^ 1][kBottomGuard + i] = e;
+      }
+      __syncthreads();
+    }
+    if (i < n) {
+      const float t = di != 0.0f ? r - row.apply(&vals[at][kBottomGuard + i], sx, sy) : 0.0f;
+      vals[at ^ 1][kBottomGuard + i] = t;
+      L.e[i] = e;
+    }
+    __syncthreads();
+    if (i < (int)C.n) {
+      int X, Y, Z;
+      node_xyz(C, (size_t)i, X, Y, Z);
+      float s = 0.0f;
+      if (C.dinv[i] != 0.0f) {
+        const int y0 = Y < 2 ? Y : 2 + C.cy * (Y - 2), y1 = Y < 2 ? Y + 1 : min(y0 + C.cy, L.ny);
+        for (int x = 2 * X; x < min(2 * X + 2, L.nx); ++x)
+          for (int y = y0; y < y1; ++y)
+            for (int z = 2 * Z; z < min(2 * Z + 2, L.nz); ++z)
+              s += vals[at ^ 1][kBottomGuard + (x * L.ny + y) * L.nz + z];
+      }
+      C.r[i] = s;
+    }
+    // (the next level writes vals[at] only; vals[at ^ 1] after its first barrier)
+  }
+  __syncthreads();
+  coarse_solve_block(G);
+  __syncthreads();
+  for (int l = lc - 1; l >= lb; --l) {
+    const TallLevel& L = G.lv[l];
+    const TallLevel& C = G.lv[l + 1];
+    const int n = (int)L.n, sy = L.nz, sx = L.ny * L.nz;
+    NodeRow<R> row;
+    float di = 0.0f, r = 0.0f, e = 0.0f;
+    if (i < n) {
+      row.load(L, K, G.reach[2 * l], G.reach[2 * l + 1], i);
+      di = L.dinv[i];
+      r = L.r[i];
+      e = L.e[i];
+      if (di != 0.0f) {
+        int x, y, z;
+        node_xyz(L, (size_t)i, x, y, z);
+        const int c = ((x >> 1) * C.ny + coarse_row(y, C.cy)) * C.nz + (z >> 1);
+        e += l + 1 == lc ? C.e[c] : vals[at][kBottomGuard + c];
+      }
+      vals[at ^ 1][kBottomGuard + i] = e;
+    }
+    at ^= 1;
+    __syncthreads();
+    for (int sw = 0; sw < kTallCoarseSweeps; ++sw, at ^= 1) {
+      if (i < n) {
+        e = di != 0.0f ? e + (r - row.apply(&vals[at][kBottomGuard + i], sx, sy)) * di : 0.0f;
+        vals[at ^ 1][kBottomGuard + i] = e;
+      }
+      __syncthreads();
+    }
+    if (l == lb && i < n) L.e2[i] = e;  // what the level above prolongs (final_e)
+  }
+}
+
 __global__ __launch_bounds__(kTallBottomThreads) void k_lat_bottom(const TallPart* parts) {
   const TallRec& G = *parts[blockIdx.x].g;
   if (G.st->done) return;
+  __shared__ BottomValues vals[2];
   const int lb = G.lb, lc = G.L - 1;
+  int reach = 0;
+  for (int l = lb; l < lc; ++l) reach = max(reach, max(G.reach[2 * l], G.reach[2 * l + 1]));
+  if (reach <= kBottomReach && lb < lc) {
+    for (int k = threadIdx.x; k < (int)(sizeof(vals) / sizeof(float)); k += blockDim.x) (&vals[0][0])[k] = 0.0f;
+    __syncthreads();
+    if (reach <= 1) bottom_in_registers<1>(G, vals);
+    else if (reach == 2) bottom_in_registers<2>(G, vals);
+    else bottom_in_registers<kBottomReach>(G, vals);
+    return;
+  }
   const int cpre = (kTallCoarseSweeps - 1) & 1;
   for (int l = lb; l < lc; ++l) {
     const int kh = G.reach[2 * l], kv = G.reach[2 * l + 1];

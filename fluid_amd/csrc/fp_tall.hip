@@ -929,7 +929,10 @@ __global__ void k_tall_true(const TallPart* parts, int np) {
 #define TALL_SEGMENTS __launch_bounds__(FP_BLOCK) __attribute__((amdgpu_waves_per_eu(5, 5)))
 
 // Block-Jacobi sweep: out = in + omega B^-1 (r - A in); first: in = 0.
-// sel: 0 reads z writes z2, 1 reads z2 writes z.
+// sel: 0 reads z writes z2, 1 reads z2 writes z.  DOT: the V-cycle's last sweep
+// also leaves r.z in the partials (a pass of its own reads both again: 15.5 us
+// at 512^2 x 34 samples and a launch, against 4 us more here).
+template <bool DOT>
 __global__ TALL_SEGMENTS void k_tall_jacobi(const TallPart* parts, int np, int sel, int first) {
   FP_PART(parts, np);
   if (G.st->done) return;
@@ -942,6 +945,7 @@ __global__ TALL_SEGMENTS void k_tall_jacobi(const TallPart* parts, int np, int s
   float* __restrict__ zout = first ? G.z : (sel ? G.z : G.z2);
   const float om = G.omega;
   const VecF zv{zin};
+  double acc[1] = {0.0};
   TALL_ITEMS(g) {
     TALL_ITEM(g, x, k, z);
     const int b = bases[g.col(x, z)], cls = G.top[g.col(x, z)];
@@ -968,13 +972,16 @@ __global__ TALL_SEGMENTS void k_tall_jacobi(const TallPart* parts, int np, int s
       for (int j = 0; j < kSegRows; ++j) {
         if (py0 + j >= g.P) break;
         const float out = first ? om * di[j] * rj[j] : ce[j] + om * di[j] * (rj[j] - ap[j]);
-        zout[g.sidx(x, py0 + j, z)] = di[j] != 0.0f ? out : 0.0f;
+        const float zn = di[j] != 0.0f ? out : 0.0f;
+        zout[g.sidx(x, py0 + j, z)] = zn;
+        if constexpr (DOT) acc[0] += (double)rj[j] * (double)zn;
       }
     } else {
       const size_t idx = g.sidx(x, 0, z);
       const fp_f32x4 inv = G.blk[g.col(x, z)];
       const size_t it = g.sidx(x, 1, z);
-      float rb = r[idx], rt = r[it];
+      const float r0b = r[idx], r0t = r[it];
+      float rb = r0b, rt = r0t;
       float ob = 0.0f, ot = 0.0f;
       if (!first) {
         float oab, oat;
@@ -984,10 +991,14 @@ __global__ TALL_SEGMENTS void k_tall_jacobi(const TallPart* parts, int np, int s
         ob = zin[idx];
         ot = zin[it];
       }
-      zout[idx] = inv.x != 0.0f || inv.y != 0.0f ? ob + om * (inv.x * rb + inv.y * rt) : 0.0f;
-      zout[it] = inv.z != 0.0f || inv.y != 0.0f ? ot + om * (inv.y * rb + inv.z * rt) : 0.0f;
+      const float zb = inv.x != 0.0f || inv.y != 0.0f ? ob + om * (inv.x * rb + inv.y * rt) : 0.0f;
+      const float zt = inv.z != 0.0f || inv.y != 0.0f ? ot + om * (inv.y * rb + inv.z * rt) : 0.0f;
+      zout[idx] = zb;
+      zout[it] = zt;
+      if constexpr (DOT) acc[0] += (double)r0b * (double)zb + (double)r0t * (double)zt;
     }
   }
+  if constexpr (DOT) block_partials<1>(acc, G.partials, blk, nblk);
 }
 
 // t = r - A z (sel: which buffer holds z).
@@ -1776,7 +1787,7 @@ int TallProjector::enqueue_vcycle(hipStream_t s, Plan& p) {
   // sample level: pre-smoothing (sweep 1 from zero writes z)
   int cur = 0;  // 0: z, 1: z2
   for (int sw = 0; sw < pre; ++sw) {
-    TTIMED(FP_KERNEL_SMOOTH_FINE, PLAUNCH(k_tall_jacobi, p.samples, s, cur, sw == 0 ? 1 : 0));
+    TTIMED(FP_KERNEL_SMOOTH_FINE, PLAUNCH(k_tall_jacobi<false>, p.samples, s, cur, sw == 0 ? 1 : 0));
     if (sw > 0) cur ^= 1;
   }
   TTIMED(FP_KERNEL_RESIDUAL_FINE, PLAUNCH(k_tall_residual, p.samples, s, cur));
@@ -1803,7 +1814,9 @@ int TallProjector::enqueue_vcycle(hipStream_t s, Plan& p) {
   }
   TTIMED(FP_KERNEL_PROLONG_FINE, PLAUNCH(k_tall_prolong0, p.samples, s, cur));
   for (int sw = 0; sw < post; ++sw) {
-    TTIMED(FP_KERNEL_SMOOTH_FINE, PLAUNCH(k_tall_jacobi, p.samples, s, cur, 0));
+    // the last sweep makes r.z of its own values
+    if (sw + 1 == post) TTIMED(FP_KERNEL_SMOOTH_FINE, PLAUNCH(k_tall_jacobi<true>, p.samples, s, cur, 0));
+    else TTIMED(FP_KERNEL_SMOOTH_FINE, PLAUNCH(k_tall_jacobi<false>, p.samples, s, cur, 0));
     cur ^= 1;
   }
   return FP_OK;
@@ -1811,7 +1824,7 @@ int TallProjector::enqueue_vcycle(hipStream_t s, Plan& p) {
 
 int TallProjector::enqueue_iteration(hipStream_t s, Plan& p) {
   enqueue_vcycle(s, p);
-  PLAUNCH(k_tall_rz, p.samples, s);
+  if (p.post == 0) PLAUNCH(k_tall_rz, p.samples, s);
   FLAUNCH(k_fin_rz<TallPart>, p.samples, s);
   TTIMED(FP_KERNEL_CG_DIRECTION, PLAUNCH(k_tall_direction, p.samples, s));
   FLAUNCH(k_fin_dq<TallPart>, p.samples, s);

@@ -50,3 +50,23 @@ def test_leg_bits(fpl, dims, precision):
             assert np.array_equal(z[0], z[1]), (sweeps, np.abs(z[0] - z[1]).max())
     finally:
         g.destroy()
+
+
+# tanks whose waves lie in air alone, in liquid alone and across a wall, an edge of a row or the surface
+@pytest.mark.parametrize("dims", [(16, 40, 64), (9, 30, 200), (20, 33, 17)])
+@pytest.mark.parametrize("fill", [0.5, 0.97])
+def test_flat_tank_matches_oracle(fpl, oracle, dims, fill):
+    rng = np.random.default_rng(dims[2])
+    h = 1.0 / max(dims)
+    y = np.arange(dims[1]) + 0.5 - fill * dims[1]
+    phi = np.broadcast_to((y * h)[None, :, None], dims).astype(np.float32).copy()
+    phi[dims[0] // 2, 1:4, :] = 0.3 * h  # a bubble line through the liquid
+    r = np.where(phi < 0, rng.standard_normal(dims), 0).astype(np.float32)
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        z = g.probe_vcycle(phi, r, precision="fp32", pre_sweeps=2, post_sweeps=2)
+        oz = oracle.vcycle(phi, r.astype(np.float64), pre=2, post=2)
+        # the bound of the 64^3 V-cycle test
+        assert np.linalg.norm(z - oz) < 2e-5 * np.linalg.norm(oz)
+    finally:
+        g.destroy()

@@ -504,7 +504,7 @@ __device__ __forceinline__ void carry_walls(const AdGeo& g, const Faces& cur, fl
 // SIMD: 128 registers; at three 2.60 ms for the 384^3 pass of a flow of one to
 // three pieces, at five the same, at six, with spills, 2.45): 3.02 -> 2.28 ms with
 // the paths by position, the first stage's few corners and the divisions by h
-// as products; 0.67 TB/s of inputs and outputs (a block order by XCD: 2.35 ms).
+// as products; 1 TB/s of inputs and outputs (a block order by XCD: 2.35 ms).
 
 // semiLagrangianAdvection (…wgsl.ts:922-936)
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_adv_sl(
@@ -554,8 +554,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 // reverseAdvection (…wgsl.ts:954-961) through the prediction's extrapolation
 // te, correctAdvection (:993-1004) with boundedMacCormack (:963-991) and the
 // forces in one pass: a face's correction needs the reverse trace of that face
-// only.  160 x 117 x 143 in MacCormack: 2.16 -> 0.98 ms with one forward trace
-// instead of two and no field of reversed or corrected faces.
+// only.  160 x 117 x 143 in MacCormack with its extrapolations: 1.18 ->
+// 0.98 ms with one forward trace instead of two and no field of reversed or
+// corrected faces.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_adv_correct(
     AdGeo g, Faces te, Faces cur, Faces pred, Faces lower, Faces upper, const float* __restrict__ phi,
     const float* __restrict__ dens, float* uo, float* vo, float* wo) {

@@ -276,7 +276,7 @@ __device__ __forceinline__ float coefficient_raw(const CmLevel& L, int i, int X,
 // the cells behind, so a stencil is one word and three floats, and neither
 // those loads nor the neighbours' pressures wait for another.  (All six
 // coefficients in 32 bytes a cell took 47.0 ms for a 256^3 projection against
-// 43.7: memory bounds the sweeps there.)
+// 43.7, both in sweeps: memory bounds them there.)
 struct CmRecord {
   float a[6], diag;
   unsigned liq;
@@ -348,10 +348,8 @@ __device__ __forceinline__ float smoothed(const float* a, float diag, unsigned l
 // from the old pressure, passes it through LDS and updates the second colour
 // of the tile, as (even z, odd z) pairs of one cell of each colour.  The ring
 // makes half the first-colour work twice, but a colour pass as a launch of its
-// own was only latency on these levels, with three loads waiting for each
-// other: a sweep of the 66^3 and 34^3 levels takes 7.0 us, its two passes took
-// 10.2 and a gap more.  At 256^3, where memory bounds it, a projection takes
-// 43.7 ms against 45.9.
+// own is only latency on small levels: a sweep of a 34^3 level takes 7.0 us, two
+// passes 8 and a gap more.  (Larger levels: kSweepCells.)
 constexpr int kSweepX = 8, kSweepY = 8, kSweepZ = 16, kSweepLanes = 512;
 __global__ __launch_bounds__(kSweepLanes) void k_cm_sweep(CmLevel L, const float* __restrict__ rhs,
                                                           const float* __restrict__ pmin) {
@@ -410,6 +408,30 @@ __global__ __launch_bounds__(kSweepLanes) void k_cm_sweep(CmLevel L, const float
   for (int nb = 0; nb < 6; ++nb) v[nb] = (r.liq >> nb & 1) ? s_first[at[nb]] : 0.0f;
   out[i] = smoothed(r.a, r.diag, r.liq, v, sr, sp, sm);
 }
+
+// The cells of one colour, in place, for the levels with more than kSweepCells:
+// there the bytes count, k_cm_sweep reads its ring's stencils twice and those of
+// air cells, and this reads an air cell's own word, pressure and p_min.
+__global__ void k_cm_colour(CmLevel L, const float* __restrict__ rhs, const float* __restrict__ pmin, int colour) {
+  CM_FOR(i, L.n) {
+    int X, Y, Z;
+    cdecode(L, i, X, Y, Z);
+    if (((X + Y + Z) & 1) != colour) continue;
+    if (!(__float_as_uint(L.coef[i].w) & kSelfLiquid)) {
+      L.p[i] = fmaxf(L.p[i], pmin[i]);
+      continue;
+    }
+    const CmRecord r = record_at(L, i, X, Y, Z);
+    float v[6];
+    neighbour_pressures(L, L.p, i, r.liq, v);
+    L.p[i] = smoothed(r.a, r.diag, r.liq, v, rhs[i], L.p[i], pmin[i]);
+  }
+}
+// Above this many padded cells: 64^3 (66^3 padded) takes 2.70 ms in colour passes
+// on its finest level and 2.99 in sweeps, 96^3 4.2 and 5.1, 384^3 at rest 85 and
+// 139 (105 with the passes and stencils of 32 bytes a neighbour); a 34^3 level
+// in colour passes too makes the 64^3 grid's 2.90.
+constexpr int kSweepCells = 1 << 17;
 
 // mgResidual (…multigrid.wgsl.ts:197-205)
 __global__ void k_cm_residual(CmLevel L, const float* __restrict__ rhs, float* __restrict__ out) {
@@ -610,9 +632,9 @@ __global__ __launch_bounds__(kCoarseLanes) void k_cm_coarse(CmLevel L, const flo
 }
 
 // mgResidual, mgRestrictResidual (…multigrid.wgsl.ts:197-215), the zero start
-// and mgDownsampleSubtract (:311-323) of the next level in one launch: a lane per coarse cell evaluates the stencils of its
-// eight children (a child away from the halo belongs to one coarse cell, so
-// hardly any residual is made twice).
+// and mgDownsampleSubtract (:311-323) of the next level in one launch: a lane per
+// coarse cell evaluates the stencils of its eight children (a child away from
+// the halo belongs to one coarse cell, so hardly any residual is made twice).
 __global__ void k_cm_descend(CmLevel F, const float* __restrict__ rhs, const float* __restrict__ fmin, int constrained,
                              CmLevel C) {
   CM_FOR(i, C.n) {
@@ -660,10 +682,10 @@ __global__ void k_cm_full_down(CmLevel F, const float* __restrict__ fmin, int co
 // and p_min in LDS, so a colour pass is a barrier instead of a launch.  On a
 // 64^3 grid 1152 of the 1560 colour passes are on these levels, and a launch
 // of one took 4 to 5 us with its gap; a V-cycle from 18^3 takes 63 us here, one
-// of 72 passes and 3 transfers, or about one us a pass.  A lane owns (even z, odd z) pairs of cells, one of each colour, and
-// holds their coefficients in registers for a whole smoothing leg.  The
-// arithmetic is that of k_cm_sweep, k_cm_descend, k_cm_full_down, k_cm_prolong
-// and k_cm_coarse.
+// of 72 passes and 3 transfers, or about one us a pass.  A lane owns (even z,
+// odd z) pairs of cells, one of each colour, and holds their coefficients in
+// registers for a whole smoothing leg.  The arithmetic is that of k_cm_sweep,
+// k_cm_descend, k_cm_full_down, k_cm_prolong and k_cm_coarse.
 // ---------------------------------------------------------------------------
 constexpr int kTailLanes = 1024;
 constexpr int kTailSlots = 3;       // pairs per lane on the first level
@@ -1151,6 +1173,11 @@ void Cm11a::tail(hipStream_t s, int full) {
 // `count` red-black sweeps; each writes the level's other pressure buffer,
 // which then is the level's pressure.
 void Cm11a::sweeps(hipStream_t s, CmLevel& c, int count, const float* rhs, const float* pmin) {
+  if (c.n > kSweepCells) {
+    for (int i = 0; i < count; ++i)
+      for (int colour = 0; colour < 2; ++colour) CM_LAUNCH(k_cm_colour, c.n, s, c, rhs, pmin, colour);
+    return;
+  }
   auto tiles = [](int n, int t) { return (n + t - 1) / t; };
   const int groups = tiles(c.D0, kSweepX) * tiles(c.D1, kSweepY) * tiles(c.D2, kSweepZ);
   for (int i = 0; i < count; ++i) {

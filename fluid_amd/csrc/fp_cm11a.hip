@@ -691,6 +691,8 @@ constexpr int kTailLanes = 1024;
 constexpr int kTailSlots = 3;       // pairs per lane on the first level
 constexpr int kTailCells = 7424;    // 16 bytes of LDS each, and 4 for the first level's residuals
 constexpr int kTailLevels = kMaxLevels;
+constexpr size_t kTailLds = (size_t)kTailCells * 20;  // beside the coarsest solve's static LDS, within a CU's 160 KB
+static_assert(kTailLds + kCoarseLanes * 8 + 256 <= 160 * 1024, "the tail fits a CU");
 
 struct CmTail {
   CmLevel lv[kTailLevels];
@@ -1120,15 +1122,15 @@ int Cm11a::create(int nx, int ny, int nz, double h) {
   if (!rc) rc = alloc((void**)&stats_, sizeof(CmStats));
   if (rc) return rc;
   // the tail starts at the first level (not the finest) whose levels fit; a
-  // device that gives a workgroup less LDS keeps one launch per pass
-  for (int l = 1; l + 1 < L && tail_ == 0; ++l) {
-    const size_t lds = tail_lds(l);
-    if (!lds) continue;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cm_tail), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) == hipSuccess)
-      tail_ = l;
-    else
-      (void)hipGetLastError();
+  // device that gives a workgroup less LDS keeps one launch per pass.  The limit
+  // belongs to the kernel on this device and not to a grid: every grid asks for
+  // the same, the most that a tail takes.
+  for (int l = 1; l + 1 < L && tail_ == 0; ++l)
+    if (tail_lds(l)) tail_ = l;
+  if (tail_ > 0 && hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cm_tail),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds) != hipSuccess) {
+    (void)hipGetLastError();
+    tail_ = 0;
   }
   return FP_OK;
 }

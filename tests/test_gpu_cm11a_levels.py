@@ -27,3 +27,19 @@ def test_levels_bit_exact(fpl, oracle, dims, sweeps, open_top):
             assert r.report["coarse_sweeps"] == orep["coarse_sweeps"]
     finally:
         g.destroy()
+
+
+def test_two_grids_alive(fpl):
+    """A second grid whose tail is smaller leaves the first one's launches as they were."""
+    scenes = [separating(d) for d in ((64, 64, 64), (16, 16, 16))]
+    grids = [fpl.UniformPressureProjection(s[0].shape, s[4]) for s in scenes]
+    try:
+        first, second = [], []
+        for out in (first, second):
+            for g, (phi, u, v, w, h, dt, rho) in zip(grids, scenes):
+                out.append(g.project(phi, u, v, w, dt, rho, solver="cm11a"))
+        for a, b in zip(first, second):
+            assert np.array_equal(a.pressure, b.pressure) and np.array_equal(a.u, b.u)
+    finally:
+        for g in grids:
+            g.destroy()

@@ -1195,27 +1195,26 @@ __global__ __launch_bounds__(kBottomThreads) void k_bottom_lds(const Part* parts
   }
 }
 
-// Most dynamic LDS of k_bottom_lds: what the device gives a workgroup beside
-// the kernel's static LDS (160 KB per CU on gfx950: 8600 cells in FP16, 6500
-// in FP32, so every bottom of a lattice that halves on all axes fits).
+// Most dynamic LDS of k_bottom_lds on the current device: what it gives a
+// workgroup beside the kernel's static LDS (160 KB per CU on gfx950: 8600 cells
+// in FP16, 6500 in FP32, so every bottom of a lattice that halves on all axes
+// fits).  A function's limit is a device's own, so each projector asks for it
+// on its context's device.
 template <typename T>
-static size_t bottom_lds_max() {
-  static const size_t most = [] {
-    const size_t fixed = sizeof(double) * kCoarseMax + 256;
-    int dev = 0, block = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-      return kBottomLdsMax;
-    const size_t want = (size_t)block > fixed ? (size_t)block - fixed : 0;
-    if (want > kBottomLdsMax &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bottom_lds<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)want) != hipSuccess) {
-      (void)hipGetLastError();
-      return kBottomLdsMax;
-    }
-    return want;
-  }();
-  return most;
+static size_t bottom_lds_grant() {
+  const size_t fixed = sizeof(double) * kCoarseMax + 256;
+  int dev = 0, block = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+    return kBottomLdsMax;
+  const size_t want = (size_t)block > fixed ? (size_t)block - fixed : 0;
+  if (want > kBottomLdsMax &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bottom_lds<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)want) != hipSuccess) {
+    (void)hipGetLastError();
+    return kBottomLdsMax;
+  }
+  return want;
 }
 
 // Packed coefficients of a fused level.  Instructions bound it where every wave
@@ -1906,7 +1905,11 @@ struct Projector::Plan {
   }
 };
 
-Projector::Projector() : noalloc_plan_(new Plan()) {}
+// (made with the context's device current)
+Projector::Projector() : noalloc_plan_(new Plan()) {
+  bottom_lds_ = std::min(bottom_lds_grant<float>(),
+                         std::min(bottom_lds_grant<__half>(), bottom_lds_grant<__hip_bfloat16>()));
+}
 
 Projector::~Projector() {
   delete noalloc_plan_;
@@ -2219,7 +2222,7 @@ int Projector::vcycle_t(hipStream_t s, Plan& p) {
     // LDS-resident bottom when its levels fit beside the static LDS (the
     // coarse solve's right-hand side)
     const size_t lds = bottom_lds_bytes_of<T>(p.bottom_n, kMaxLevels);
-    if (lds <= bottom_lds_max<T>())
+    if (lds <= bottom_lds_)
       hipLaunchKernelGGL((k_bottom_lds<T>), dim3(p.coarse_deep.n), dim3(kBottomThreads), lds, s, p.coarse_deep.dev,
                          pre, post);
     else

@@ -25,7 +25,7 @@ namespace fp {
 constexpr int kMaxLevels = 16;
 constexpr unsigned kMaxBlocks = 16384;
 // Dynamic LDS that the LDS-resident V-cycle bottom (k_bottom_lds) takes on
-// any device; bottom_lds_max asks for more.
+// any device; a projector asks for more (bottom_lds_grant).
 constexpr size_t kBottomLdsMax = 48 * 1024;
 constexpr long long kBottomCells = 4096;  // levels below this size run in the one-workgroup bottom of the V-cycle
 constexpr int kBottomThreads = 1024;
@@ -315,6 +315,7 @@ class Projector {
   void timer_end(hipStream_t s);
   std::map<std::vector<long long>, Plan*> plans_;
   Plan* noalloc_plan_ = nullptr;  // host tables of run_noalloc
+  size_t bottom_lds_ = kBottomLdsMax;  // most dynamic LDS of k_bottom_lds on the context's device
   int timed_kernel_ = 0;
   int timer_used_ = 0;
   std::vector<hipEvent_t> timer_events_;

@@ -240,6 +240,13 @@ struct Uniform {
     fp_report r;
     return FP(fp_project)(g, &in, &out, &o, &r);
   }
+  int vcycle(int precision) {
+    fp_options o;
+    must(FP(fp_default_options)(&o), "fp_default_options");
+    o.precision = precision;
+    std::vector<float> z(phi.size());
+    return FP(fp_probe_vcycle)(g, phi.data(), &o, phi.data(), z.data());
+  }
   void destroy() { must(FP(fp_grid_destroy)(g), "fp_grid_destroy"); }
 };
 
@@ -266,6 +273,20 @@ void cm11a_two_grids() {
   must(FP(fp_ctx_destroy)(c), "fp_ctx_destroy");
 }
 
+// The same FP32 grid, its V-cycle's bottom above 64 KB, on a context per device.
+void two_devices() {
+  fp_ctx* c[kDevices];
+  for (int d = 0; d < kDevices; ++d) c[d] = context(d);
+  for (int round = 0; round < 2; ++round)
+    for (int d = 0; d < kDevices; ++d) {
+      Uniform g(c[d], 30, 30, 30);
+      must(g.vcycle(FP_PRECISION_FP32), "30^3");
+      g.destroy();
+    }
+  must_launch("k_bottom_lds");
+  for (fp_ctx* x : c) must(FP(fp_ctx_destroy)(x), "fp_ctx_destroy");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -273,7 +294,8 @@ int main(int argc, char** argv) {
     std::printf("usage: launches LIBRARY SCENARIO... (%s)\n", argc < 3 ? "arguments" : dlerror());
     return 99;
   }
-  const std::map<std::string, void (*)()> scenarios{{"cm11a_two_grids", cm11a_two_grids}};
+  const std::map<std::string, void (*)()> scenarios{{"cm11a_two_grids", cm11a_two_grids},
+                                                        {"two_devices", two_devices}};
   for (int k = 2; k < argc; ++k) scenarios.at(argv[k])();
   std::printf("%d wrong\n", g_wrong);
   std::fflush(stdout);

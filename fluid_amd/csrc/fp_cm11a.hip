@@ -1060,7 +1060,7 @@ size_t Cm11a::estimate_bytes(int nx, int ny, int nz) {
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   for (int l = 0; l < L; ++l) {
     const size_t n = (size_t)(dims[l][0] + 2) * (dims[l][1] + 2) * (dims[l][2] + 2);
-    total += 7 * up(n * 4) + 2 * up(n * 16);
+    total += (n > kSweepCells ? 6 : 7) * up(n * 4) + 2 * up(n * 16);
     if (l == 0) total += 4 * up(n * 4);
   }
   return total + up((size_t)kMeasureBlocks * 16) + up(sizeof(CmStats));
@@ -1107,7 +1107,7 @@ int Cm11a::create(int nx, int ny, int nz, double h) {
     if (!rc) rc = alloc((void**)&c.topo, b16);
     if (!rc) rc = alloc((void**)&c.coef, b16);
     if (!rc) rc = alloc((void**)&c.p, b4);
-    if (!rc) rc = alloc((void**)&c.p2, b4);
+    if (!rc && c.n <= kSweepCells) rc = alloc((void**)&c.p2, b4);  // k_cm_colour works in place
     if (!rc) rc = alloc((void**)&c.rhs0, b4);
     if (!rc) rc = alloc((void**)&c.rhs1, b4);
     if (!rc) rc = alloc((void**)&c.pmin, b4);

@@ -30,7 +30,8 @@ struct CmLevel {
   float4* topo;    // cell dual volume, +x/+y/+z face dual volumes
   float4* coef;    // +x/+y/+z coefficients V / (h^2 theta), liquid flags of the cell and its neighbours
   float* p;        // pressure
-  float* p2;       // the buffer that the next sweep writes (they then change places)
+  float* p2;       // the buffer that the next sweep writes (they then change places); none where colour
+                   // passes work in place
   float* rhs0;     // V-cycle right-hand side
   float* rhs1;     // full-cycle correction right-hand side
   float* pmin;     // p_min of the level

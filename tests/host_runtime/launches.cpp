@@ -273,6 +273,32 @@ void cm11a_two_grids() {
   must(FP(fp_ctx_destroy)(c), "fp_ctx_destroy");
 }
 
+// A finest level whose passes work in place holds no second pressure, and the
+// bytes that a call is refused by are those it takes.
+void cm11a_bytes() {
+  const size_t n = 98, level = (n * n * n * 4 + 255) & ~(size_t)255;  // 96^3 with its halo
+  fp_ctx* c = context(0);
+  Uniform g(c, 96, 96, 96);
+  const std::map<void*, size_t> before = g_blocks;
+  must(g.project(FP_SOLVER_CM11A, FP_PRECISION_MIXED_FP16), "96^3");
+  int arrays = 0;
+  for (const auto& b : g_blocks) arrays += before.count(b.first) == 0 && b.second == level;
+  // level sets, pressure, right-hand sides, p_min; b, p_min, its shift and the backup
+  if (arrays != 10) wrong(std::to_string(arrays) + " arrays of the finest level, 10 expected");
+  uint64_t used = 0;
+  must(FP(fp_ctx_bytes_in_use)(c, &used), "fp_ctx_bytes_in_use");
+  g.destroy();
+  must(FP(fp_ctx_destroy)(c), "fp_ctx_destroy");
+  for (int less = 0; less < 2; ++less) {
+    fp_ctx* b = context(0, used - less);
+    Uniform q(b, 96, 96, 96);
+    const int rc = q.project(FP_SOLVER_CM11A, FP_PRECISION_MIXED_FP16);
+    if (rc != (less ? FP_ERR_BUDGET : FP_OK)) wrong("budget of " + std::to_string(used - less) + ": " + std::to_string(rc));
+    q.destroy();
+    must(FP(fp_ctx_destroy)(b), "fp_ctx_destroy");
+  }
+}
+
 // The same FP32 grid, its V-cycle's bottom above 64 KB, on a context per device.
 void two_devices() {
   fp_ctx* c[kDevices];
@@ -294,7 +320,8 @@ int main(int argc, char** argv) {
     std::printf("usage: launches LIBRARY SCENARIO... (%s)\n", argc < 3 ? "arguments" : dlerror());
     return 99;
   }
-  const std::map<std::string, void (*)()> scenarios{{"cm11a_two_grids", cm11a_two_grids},
+  const std::map<std::string, void (*)()> scenarios{{"cm11a_bytes", cm11a_bytes},
+                                                        {"cm11a_two_grids", cm11a_two_grids},
                                                         {"two_devices", two_devices}};
   for (int k = 2; k < argc; ++k) scenarios.at(argv[k])();
   std::printf("%d wrong\n", g_wrong);

@@ -649,17 +649,21 @@ int fp_probe_taps(fp_grid* g, int32_t level, int32_t axis, int32_t* prolong_coar
                         restrict_weight);
 }
 
-// The grid's extrapolation state, created on first use within the context's budget.
-static int ensure_extrapolator(fp_grid* g, const char* what) {
-  if (g->extrap) return FP_OK;
+// The grid's extrapolation state, created on first use within the context's
+// budget; host: with the staging of a host-memory extrapolation.
+static int ensure_extrapolator(fp_grid* g, const char* what, bool host) {
+  const bool staged = !host || (g->extrap && g->extrap->host_ready());
+  if (g->extrap && staged) return FP_OK;
   fp_ctx* ctx = g->ctx;
   const fp_grid_desc& d = g->desc;
-  const uint64_t need = fp::Extrapolator::estimate_bytes(d.nx, d.ny, d.nz);
+  const uint64_t need = (g->extrap ? 0 : fp::Extrapolator::estimate_bytes(d.nx, d.ny, d.nz)) +
+                        (staged ? 0 : fp::Extrapolator::host_bytes(d.nx, d.ny, d.nz));
   if (ctx->budget && ctx->in_use + need > ctx->budget) {
     set_error("%s: %llu more bytes exceed the context's HBM budget (%llu of %llu in use)", what,
               (unsigned long long)need, (unsigned long long)ctx->in_use, (unsigned long long)ctx->budget);
     return FP_ERR_BUDGET;
   }
+  if (g->extrap) return FP_OK;
   fp::Extrapolator* e = new (std::nothrow) fp::Extrapolator();
   if (!e) return FP_ERR_OUT_OF_MEMORY;
   int rc = e->create(d.nx, d.ny, d.nz, d.h);
@@ -685,9 +689,12 @@ int fp_extrapolate_velocity(fp_grid* g, const fp_extrapolate_args* a, fp_extrapo
   fp_ctx* ctx = g->ctx;
   std::lock_guard<std::mutex> lock(ctx->gpu);
   (void)hipSetDevice(ctx->device);
-  int rc = ensure_extrapolator(g, "fp_extrapolate_velocity");
+  int rc = ensure_extrapolator(g, "fp_extrapolate_velocity", a->memory == FP_MEMORY_HOST);
   if (rc) return rc;
-  return g->extrap->run(ctx->stream, a, rep);
+  const size_t before = g->extrap->bytes();
+  rc = g->extrap->run(ctx->stream, a, rep);
+  ctx->in_use += g->extrap->bytes() - before;  // host staging, on the first host-memory call
+  return rc;
 }
 
 int fp_advect_velocity(fp_grid* g, const fp_advect_args* a, fp_advect_report* rep) {
@@ -708,7 +715,7 @@ int fp_advect_velocity(fp_grid* g, const fp_advect_args* a, fp_advect_report* re
   fp_ctx* ctx = g->ctx;
   std::lock_guard<std::mutex> lock(ctx->gpu);
   (void)hipSetDevice(ctx->device);
-  int rc = ensure_extrapolator(g, "fp_advect_velocity");
+  int rc = ensure_extrapolator(g, "fp_advect_velocity", false);
   if (rc) return rc;
   if (!g->advect) {
     const fp_grid_desc& d = g->desc;

@@ -6,9 +6,10 @@
 // (L1) distance to every source face exceeds 3 never activates, since each
 // Godunov step adds at least h/sqrt(3) and the band ends at 2h, so after the
 // seed three dilations of the source masks and one compaction give the list
-// of cells the passes visit; cells off the list keep their seed state, which
-// the seed writes to both ping-pong sides.  Each pass is one launch over the
-// list that returns at once when an earlier pass left no face active (the
+// of cells the passes visit.  The seed writes the whole state, on both
+// ping-pong sides, at those cells and their neighbours; elsewhere only side A's
+// known flags and known values, and nothing else there may be read.  Each pass is
+// one launch over the list that returns at once when an earlier pass left no face active (the
 // reference's indirect dispatch chain).  The hierarchy and the seed stream
 // the whole grid in XCD-contiguous chunks.  No contraction anywhere: results
 // equal oracle/fp_oracle_extrap.c bit for bit.
@@ -940,9 +941,8 @@ size_t Extrapolator::estimate_bytes(int nx, int ny, int nz) {
   auto round = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t n = (size_t)nx * ny * nz;
   const size_t padded = n + 2 * quad_pad(ny, nz);
-  size_t total = 2 * 6 * round(n * 4) + 4 * round(n) + 3 * round(padded) + round(n * 4) +
-                 round(sizeof(ExCounters)) + round(sizeof(ExTotals));
-  total += round(n * 4) + round(((size_t)(nx + 1) * ny * nz + (size_t)nx * (ny + 1) * nz + (size_t)nx * ny * (nz + 1)) * 4);
+  size_t total = 2 * 6 * round(n * 4) + 3 * round(n) + 3 * round(padded) + round(n * 4) +
+                 round(sizeof(ExCounters) + sizeof(ExTotals));
   std::vector<std::array<int, 3>> dims;
   level_dims(nx, ny, nz, &dims);
   for (const auto& d : dims) {
@@ -966,18 +966,17 @@ int Extrapolator::create(int nx, int ny, int nz, double h) {
       if ((rc = alloc((void**)&st_[k].dist[c], n * 4))) return rc;
     }
     if ((rc = alloc((void**)&st_[k].flags, n))) return rc;
-    if ((rc = alloc((void**)&st_[k].stat, n))) return rc;
   }
+  if ((rc = alloc((void**)&st_[1].stat, n))) return rc;
   const size_t pad = quad_pad(ny, nz);
   for (uint8_t** p : {&cls_, &cand_[0], &cand_[1]}) {
     if ((rc = alloc((void**)p, n + 2 * pad))) return rc;
     *p += pad;
   }
+  st_[0].stat = cand_[0];  // the last dilation is its last reader, the seed this one's first writer
   if ((rc = alloc((void**)&list_, n * 4))) return rc;
-  if ((rc = alloc((void**)&counters_, sizeof(ExCounters)))) return rc;
-  if ((rc = alloc((void**)&totals_, sizeof(ExTotals)))) return rc;
-  const size_t faces = (size_t)(nx + 1) * ny * nz + (size_t)nx * (ny + 1) * nz + (size_t)nx * ny * (nz + 1);
-  if ((rc = alloc((void**)&in_, n * 4 + faces * 4))) return rc;
+  if ((rc = alloc((void**)&counters_, sizeof(ExCounters) + sizeof(ExTotals)))) return rc;
+  totals_ = reinterpret_cast<ExTotals*>(counters_ + 1);
   std::vector<std::array<int, 3>> dims;
   level_dims(nx, ny, nz, &dims);
   for (const auto& d : dims) {
@@ -998,6 +997,13 @@ int Extrapolator::create(int nx, int ny, int nz, double h) {
   return FP_OK;
 }
 
+int Extrapolator::stage_host() { return in_ ? FP_OK : alloc((void**)&in_, host_bytes(d_[0], d_[1], d_[2])); }
+
+size_t Extrapolator::host_bytes(int nx, int ny, int nz) {
+  const size_t faces = (size_t)(nx + 1) * ny * nz + (size_t)nx * (ny + 1) * nz + (size_t)nx * ny * (nz + 1);
+  return (faces * 4 + 255) & ~(size_t)255;
+}
+
 int Extrapolator::run(hipStream_t s, const fp_extrapolate_args* a, fp_extrapolate_report* rep, bool same_band) {
   const auto t0 = std::chrono::steady_clock::now();
   const int nx = d_[0], ny = d_[1], nz = d_[2];
@@ -1014,8 +1020,10 @@ int Extrapolator::run(hipStream_t s, const fp_extrapolate_args* a, fp_extrapolat
   // staging (free once the seed has read the inputs) and are copied back
   float *uo = a->u_out, *vo = a->v_out, *wo = a->w_out;
   if (a->memory == FP_MEMORY_HOST) {
-    float* f = in_;
-    float* hu = f + n;
+    const int rc = stage_host();
+    if (rc) return rc;
+    float* f = st_[1].val[0];  // read by the classification only, written by the seed after it
+    float* hu = in_;
     float* hv = hu + nu;
     float* hw = hv + nv;
     HIPCHK(hipMemcpyAsync(f, field, (size_t)n * 4, hipMemcpyHostToDevice, s));

@@ -57,7 +57,10 @@ struct ExTotals {
 class Extrapolator {
  public:
   ~Extrapolator();
+  // Bytes of create(), and those that the first host-memory run adds.
   static size_t estimate_bytes(int nx, int ny, int nz);
+  static size_t host_bytes(int nx, int ny, int nz);
+  bool host_ready() const { return in_ != nullptr; }
   int create(int nx, int ny, int nz, double h);
   // One extrapolation of a->phi / a->density and a->u, a->v, a->w into the
   // outputs; synchronous on s.
@@ -69,6 +72,7 @@ class Extrapolator {
 
  private:
   int alloc(void** p, size_t bytes);
+  int stage_host();
   std::vector<void*> allocations_;
   std::vector<ExLevel> levels_;
   size_t bytes_ = 0;
@@ -80,9 +84,9 @@ class Extrapolator {
   uint8_t* cand_[2] = {nullptr, nullptr};
   int band_count_ = -1;  // band list length of the previous run (-1: none)
   int* list_ = nullptr;
-  float* in_ = nullptr;  // host-memory staging: phi or density, u, v, w
+  float* in_ = nullptr;  // host-memory staging of u, v, w
   ExCounters* counters_ = nullptr;
-  ExTotals* totals_ = nullptr;
+  ExTotals* totals_ = nullptr;  // behind the counters
 };
 
 }  // namespace fp

@@ -348,8 +348,8 @@ int fp_tall_remesh(fp_grid* grid, const fp_tall_remesh_args* args, int64_t* chan
  * unknown).  Outputs: known values on open faces, 0 on walls and on open
  * faces the hierarchy leaves unknown (packTransportShell, :491-512).  FP32.
  * Outputs may alias the inputs.  The first call on a grid allocates the
- * extrapolation state (about 59 bytes per cell; FP_ERR_BUDGET beyond the
- * context's budget).  Device arrays must be complete when the call is made;
+ * extrapolation state (about 62 bytes per cell) and the first one in host
+ * memory its staging (12 more); FP_ERR_BUDGET beyond the context's budget.  Device arrays must be complete when the call is made;
  * it returns when the outputs are written. */
 typedef struct {
   int32_t memory;       /* FP_MEMORY_HOST or FP_MEMORY_DEVICE for the arrays below */

@@ -27,6 +27,8 @@ constexpr int kDevices = 2;
 constexpr int kBlockLds = 160 * 1024;    // gfx950
 constexpr size_t kUngranted = 64 * 1024; // dynamic LDS of a function whose limit was never raised
 
+constexpr size_t kCounters = 24 * 1024;  // of an extrapolation, spread over cache lines
+
 int g_wrong = 0;
 thread_local int g_device = 0;
 std::map<const void*, std::string> g_functions;
@@ -299,6 +301,50 @@ void cm11a_bytes() {
   }
 }
 
+// An extrapolation's state and host staging stay within 48 bytes a cell for two
+// sides of values and distances, 5 for flags, classes and masks, 4 for the list,
+// 4 a cell and 4 a face for host arrays, and the hierarchy: budgets that held
+// those hold the call.
+void extrapolate_bytes() {
+  const int shapes[][3] = {{2, 40, 33}, {33, 2, 40}, {16, 16, 16}, {48, 31, 50}};
+  for (const auto& d : shapes)
+    for (int memory = 0; memory < 2; ++memory)
+      for (int pass = 0; pass < 2; ++pass) {  // without a budget, then with that one
+        const size_t nx = d[0], ny = d[1], nz = d[2], n = nx * ny * nz;
+        auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+        const size_t faces = (nx + 1) * ny * nz + nx * (ny + 1) * nz + nx * ny * (nz + 1);
+        size_t most = 13 * up(4 * n) + 5 * up(n) + up(4 * n) + up(4 * faces) + 256;
+        for (size_t a = nx, b = ny, c = nz; a > 1 && b > 1 && c > 1;) {
+          a = (a + 1) / 2;
+          b = (b + 1) / 2;
+          c = (c + 1) / 2;
+          most += 6 * up(4 * a * b * c) + 2 * up(a * b * c);
+        }
+        static uint64_t grid;  // of the pass before
+        fp_ctx* c = context(0, pass ? grid + most + kCounters : 0);
+        Uniform g(c, d[0], d[1], d[2]);
+        must(FP(fp_ctx_bytes_in_use)(c, &grid), "fp_ctx_bytes_in_use");
+        fp_extrapolate_args a;
+        std::memset(&a, 0, sizeof(a));
+        a.memory = memory;
+        a.phi = g.phi.data();
+        a.u = a.u_out = g.u.data();
+        a.v = a.v_out = g.v.data();
+        a.w = a.w_out = g.w.data();
+        const std::string what = std::to_string(nx) + "x" + std::to_string(ny) + "x" + std::to_string(nz) +
+                                 (memory == FP_MEMORY_HOST ? " host" : " device");
+        for (int call = 0; call < 2; ++call) must(FP(fp_extrapolate_velocity)(g.g, &a, nullptr), what.c_str());
+        uint64_t used = 0;
+        must(FP(fp_ctx_bytes_in_use)(c, &used), "fp_ctx_bytes_in_use");
+        if (pass && used > grid + most + kCounters)
+          wrong(what + ": " + std::to_string(used - grid) + " bytes, at most " + std::to_string(most));
+        g.destroy();
+        must(FP(fp_ctx_bytes_in_use)(c, &used), "fp_ctx_bytes_in_use");
+        if (used != 0) wrong(what + ": " + std::to_string(used) + " bytes in use after the grid");
+        must(FP(fp_ctx_destroy)(c), "fp_ctx_destroy");
+      }
+}
+
 // The same FP32 grid, its V-cycle's bottom above 64 KB, on a context per device.
 void two_devices() {
   fp_ctx* c[kDevices];
@@ -322,6 +368,7 @@ int main(int argc, char** argv) {
   }
   const std::map<std::string, void (*)()> scenarios{{"cm11a_bytes", cm11a_bytes},
                                                         {"cm11a_two_grids", cm11a_two_grids},
+                                                        {"extrapolate_bytes", extrapolate_bytes},
                                                         {"two_devices", two_devices}};
   for (int k = 2; k < argc; ++k) scenarios.at(argv[k])();
   std::printf("%d wrong\n", g_wrong);

@@ -23,7 +23,7 @@ def launches(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["cm11a_bytes", "cm11a_two_grids", "two_devices"])
+@pytest.mark.parametrize("scenario", ["cm11a_bytes", "cm11a_two_grids", "extrapolate_bytes", "two_devices"])
 def test_host_side(launches, scenario):
     r = subprocess.run([launches, build.LIB, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]

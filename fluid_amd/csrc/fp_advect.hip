@@ -34,6 +34,8 @@ struct AdGeo {
   float dt, gravity, nu;
 };
 
+constexpr float kTinyCell = 1e-22f;  // smaller cells divide (div_h)
+
 struct Faces {
   const float* f[3];
 };
@@ -74,9 +76,10 @@ __device__ __forceinline__ unsigned fidx(const AdGeo& g, int c, int x, int y, in
 // (Markstein 1990: the first quotient is within 1.5 ulp, the second faithful,
 // the third rounded as the division) in five full-rate operations, where the
 // division takes eleven and a quarter-rate reciprocal, 21 times a cell and
-// step.  A quotient so small that its residual underflows never reaches a
-// position of 1/2 or more, and zero keeps its value, not its sign (subtracted
-// or compared only).  For |x| < g.far: beyond it a quotient may overflow.
+// step.  A residual, 2^-48 of x, underflows for quotients below 2^-101 / h: with
+// h of kTinyCell or more those never reach a position of 1/2 or more, and zero
+// keeps its value, not its sign (subtracted or compared only).  For |x| < g.far:
+// beyond it a quotient may overflow.
 __device__ __forceinline__ float div_h(const AdGeo& g, float x) {
   const float q0 = x * g.inv_h;
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, g.h, x), g.inv_h, q0);
@@ -714,7 +717,7 @@ int Advector::run(hipStream_t s, Extrapolator* ex, const fp_advect_args* a, fp_a
   g.d[2] = nz;
   g.h = h_;
   g.inv_h = 1.0f / h_;
-  g.far = std::isnormal(h_) && std::isnormal(g.inv_h) ? std::min(1e38f * h_, 3e38f) : 0.0f;
+  g.far = h_ >= kTinyCell && std::isnormal(g.inv_h) ? std::min(1e38f * h_, 3e38f) : 0.0f;
   g.open_top = open_top;
   g.no_slip = a->no_slip ? 1 : 0;
   g.dt = (float)a->dt;

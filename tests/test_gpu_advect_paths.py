@@ -33,3 +33,24 @@ def test_paths_bit_exact(fpl, oracle, dims, scheme):
                 assert np.array_equal(a, b, equal_nan=True), (cells, top)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("h", [3e-36, 7e-34, 2e-31, 5e-29, 3e-27, 1e-24, 1e-20])
+def test_tiny_cells(fpl, oracle, h):
+    """Cell sizes at which a residual of the quotient by h, 2^-48 of the dividend, is subnormal."""
+    dims = (9, 12, 33)
+    rng = np.random.default_rng(4)
+    phi = np.full(dims, -h, np.float32)
+    shapes = [(dims[0] + (a == 0), dims[1] + (a == 1), dims[2] + (a == 2)) for a in range(3)]
+    field = [(rng.standard_normal(s) * 0.7 * h).astype(np.float32) for s in shapes]
+    cur = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        want = oracle.advect_velocity(*cur, h, 1.0, phi=phi, transport=field, gravity=0.0, nu=0.0,
+                                      scheme="semi-lagrangian", open_top=0)
+        got = g.advect(*cur, 1.0, phi=phi, transport=field, gravity=0.0, viscosity=0.0, scheme="semi-lagrangian",
+                       open_top=False)
+        for a, b in zip(got[:3], want):
+            assert np.array_equal(a, b, equal_nan=True)
+    finally:
+        g.destroy()

@@ -54,3 +54,36 @@ def test_tiny_cells(fpl, oracle, h):
             assert np.array_equal(a, b, equal_nan=True)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("dims", [(3, 2, 130), (12, 20, 64), (21, 18, 33)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_non_finite_transport(fpl, oracle, dims, value):
+    """A wave that meets a face that is not finite samples its first stage in
+    full (0 times an infinity is not 0).  Its faces out of reach of that one,
+    more than three cells away in a flow of a third of a cell, keep the bits of
+    the finite field.  (What a face in reach becomes is not compared: clamps
+    of a NaN differ between the device and C.)"""
+    rng = np.random.default_rng(sum(dims))
+    h, dt = 1.0 / max(dims), 0.01
+    y = np.arange(dims[1]) + 0.5
+    phi = np.broadcast_to((y - 0.6 * dims[1])[None, :, None] * h, dims).astype(np.float32).copy()
+    shapes = [(dims[0] + (a == 0), dims[1] + (a == 1), dims[2] + (a == 2)) for a in range(3)]
+    field = [(rng.uniform(-0.33, 0.33, s) * h / dt).astype(np.float32) for s in shapes]
+    cur = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    options = dict(phi=phi, gravity=-9.81, scheme="semi-lagrangian")
+    want = oracle.advect_velocity(*cur, h, dt, transport=field, nu=0.0, open_top=0, **options)
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        for c in range(3):
+            at = tuple(int(rng.integers(0, n)) for n in shapes[c])
+            broken = [f.copy() for f in field]
+            broken[c][at] = value
+            got = g.advect(*cur, dt, transport=broken, viscosity=0.0, open_top=False, **options)
+            for a, b in zip(got[:3], want):
+                d = np.max([np.abs(np.arange(n) - q).reshape([-1 if k == j else 1 for j in range(3)]) * np.ones(a.shape)
+                            for k, (n, q) in enumerate(zip(a.shape, at))], axis=0)
+                assert np.array_equal(a[d > 3], b[d > 3]), (c, at)
+            assert not all(np.array_equal(a, b) for a, b in zip(got[:3], want)), (c, at)
+    finally:
+        g.destroy()

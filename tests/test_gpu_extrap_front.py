@@ -47,3 +47,17 @@ def test_front_bit_exact(fpl, oracle, dims, open_top):
     finally:
         if g:
             g.destroy()
+
+
+# the first coarse level above the size that takes tiles, odd itself and no multiple of a tile on any axis
+@pytest.mark.parametrize("dims", [(205, 213, 209)])
+def test_tiled_levels_bit_exact(fpl, oracle, dims):
+    phi, vel, h = surface(dims, 3, "rough")
+    g = fpl.UniformPressureProjection(dims, h)
+    try:
+        want = oracle.extrapolate(*vel, h, phi=phi)
+        got = g.extrapolate(*vel, phi=phi)
+        for a, b in zip(got[:3], want[:3]):
+            assert np.array_equal(a, b)
+    finally:
+        g.destroy()

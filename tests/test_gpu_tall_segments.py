@@ -53,13 +53,16 @@ def test_segments_match_oracle(fpl, oracle, nx, nz, ny, band, depth, rough, slop
         g.destroy()
 
 
-@pytest.mark.parametrize("nx,nz,ny,band,delta", [(16, 12, 40, 8, 1), (20, 9, 40, 8, 4), (2, 40, 40, 8, 4),
-                                                 (18, 14, 90, 16, 8), (13, 21, 120, 20, 11), (40, 3, 60, 9, 6)])
-def test_small_lattice_levels(fpl, oracle, nx, nz, ny, band, delta):
+@pytest.mark.parametrize("nx,nz,ny,band,delta,iterations", [
+    (16, 12, 40, 8, 1, 13), (20, 9, 40, 8, 4, 13), (2, 40, 40, 8, 4, 14), (18, 14, 90, 16, 8, 16),
+    (13, 21, 120, 20, 11, 17), (40, 3, 60, 9, 6, 16)])
+def test_small_lattice_levels(fpl, oracle, nx, nz, ny, band, delta, iterations):
     """Levels that run in one workgroup, for couplings of one row's reach to
-    eight.  The V-cycle reduces the residual about tenfold (8 iterations to
-    1e-6 at delta 4); one whose small levels are wrong is no better than the
-    levels above them alone."""
+    eight.  Outer refinement corrects any V-cycle, so a wrong small level shows
+    in the iterations alone: those of a right one to 1e-8 are given with the case, as
+    measured; other right-hand sides of the same shapes take one more or two, a
+    V-cycle with one sweep a side less four to eight.  The pressure is the
+    oracle's to FP32's rounding of it (2.5e-8, measured too)."""
     sc = scenes.tall_random_scene(nx, nz, ny, band, seed=nx + delta, max_delta=delta)
     t = oracle.Tall(sc.layout.bases, sc.phi, sc.layout.fine_ny, sc.layout.band, sc.layout.h, sc.layout.max_delta)
     want = t.projection(sc.u, sc.v, sc.w, sc.dt, sc.rho, rel_tol=1e-12)[0]
@@ -67,7 +70,7 @@ def test_small_lattice_levels(fpl, oracle, nx, nz, ny, band, delta):
     try:
         got = g.project(sc.phi, sc.u, sc.v, sc.w, sc.dt, sc.rho, relative_tolerance=1e-8)
         print(got.report["iterations"], got.report["levels"])
-        assert got.report["relative_residual"] <= 1e-8 and got.report["iterations"] <= 30
-        assert np.linalg.norm(got.pressure - want) <= 1e-5 * np.linalg.norm(want)
+        assert got.report["relative_residual"] <= 1e-8 and got.report["iterations"] <= iterations + 2
+        assert np.linalg.norm(got.pressure - want) <= 1e-7 * np.linalg.norm(want)
     finally:
         g.destroy()

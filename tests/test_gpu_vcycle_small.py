@@ -35,9 +35,11 @@ def test_bottom_matches_oracle(fpl, oracle, dims):
         g.destroy()
 
 
-# one tile, ragged tiles, axes that do not coarsen, an odd row length, and both sides of the size limit of FP32 legs
+# one tile, ragged tiles, axes that do not coarsen, an odd row length, and both sides of the size limits of the legs (FP32,
+# then two-byte storage)
 @pytest.mark.parametrize("dims", [(16, 16, 16), (4, 16, 64), (17, 19, 23), (33, 20, 18), (40, 24, 17), (5, 33, 32),
-                                  (64, 10, 21), (80, 81, 80), (81, 81, 81)])
+                                  (64, 10, 21), (80, 81, 80), (81, 81, 81), (101, 101, 102),
+                                  (102, 101, 102)])
 @pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
 def test_leg_bits(fpl, dims, precision):
     phi, r, h = blob_case(dims, sum(dims))

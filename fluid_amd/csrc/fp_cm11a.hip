@@ -430,7 +430,9 @@ __global__ void k_cm_colour(CmLevel L, const float* __restrict__ rhs, const floa
 // Above this many padded cells: 64^3 (66^3 padded) takes 2.70 ms in colour passes
 // on its finest level and 2.99 in sweeps, 96^3 4.2 and 5.1, 384^3 at rest 85 and
 // 139 (105 with the passes and stencils of 32 bytes a neighbour); a 34^3 level
-// in colour passes too makes the 64^3 grid's 2.90.
+// in colour passes too makes the 64^3 grid's 2.90.  Between: 32 x 64 x 64 (148 K
+// padded) 2.53 either way, 48 x 48 x 96 (245 K) 2.79 and 3.04; the grids of 76 K and
+// 125 K, in sweeps on every level, 2.28 and 2.48, in colour passes 2.60 and 2.74.
 constexpr int kSweepCells = 1 << 17;
 
 // mgResidual (…multigrid.wgsl.ts:197-205)

@@ -442,8 +442,8 @@ __device__ __forceinline__ float upwind(const ExGeo& g, const float* nd, const f
 // keeps as kEligible, on the converged neighbour's new distance, which is
 // that neighbour's state, and on its own distance, which did not change.  So
 // a face reads its six neighbours and nothing further, where one of seven
-// Godunov updates was its own before: 90 -> 41 us a pass on the 654 K cells
-// under 384^3, 39 -> 9.4 us at 160 x 117 x 143.
+// Godunov updates was its own before: 90 -> 33 us a pass on the 654 K cells
+// under 384^3, 39 -> 8.3 us at 160 x 117 x 143.
 //
 // The pass therefore counts the faces active before it; `last` only counts
 // (the faces that the pass before left active).  A wave takes one component of
@@ -780,7 +780,7 @@ __device__ __forceinline__ bool tile_of(const int* T, int& x0, int& y0, int& z0)
 
 // prolongUnknownVelocity (…wgsl.ts:473-488) into a level's up arrays, a lane
 // per cell: for levels too small to fill the chip with tiles, where a tile's
-// staging is one more round trip (0.34 M cells: 11.6 us, 15.9 in tiles)
+// staging is one more round trip (kTileCells)
 __global__ __launch_bounds__(kThreads) void k_ex_prolong_cells(ExSrc src, ExLevel tgt, FastDiv tz, FastDiv ty) {
   const unsigned n = (unsigned)tgt.n;
   const unsigned i = chunk_of((n + kThreads - 1) / kThreads) * kThreads + threadIdx.x;
@@ -801,9 +801,14 @@ __global__ __launch_bounds__(kThreads) void k_ex_prolong_cells(ExSrc src, ExLeve
   }
   tgt.up_known[i] = (uint8_t)known;
 }
-constexpr long long kTileCells = 1 << 20;  // levels of this many cells take tiles
+// Levels of this many cells take tiles.  A lane per cell against tiles, cubic
+// levels: 48^3 7.0 / 8.3 us, 64^3 8.2 / 8.6, 72^3 10.2 / 9.8, 80^3 12.0 / 12.1, 88^3
+// 15.4 / 13.8, 96^3 17.3 / 15.9, 104^3 (1.1 M) 21.7 / 20.2, 128^3 34.8 / 25.1; 80 x 59 x
+// 72, whose last tiles are thin, 11.6 / 15.9.  Between 0.4 and 1 M cells the two
+// are within 1.6 us on cubes and tiles lose where they divide a level badly.
+constexpr long long kTileCells = 1 << 20;
 
-// The same in tiles: 113 us -> 74 on the 192^3 level.
+// The same in tiles: 113 us -> 70 on the 192^3 level.
 __global__ __launch_bounds__(kThreads) void k_ex_prolong(ExSrc src, ExLevel tgt) {
   __shared__ float2 win[3 * kWin];
   int x0, y0, z0;
@@ -835,8 +840,9 @@ __global__ __launch_bounds__(kThreads) void k_ex_prolong(ExSrc src, ExLevel tgt)
 
 // the last prolongation onto the band result, packed into the face arrays
 // (packTransportShell, …wgsl.ts:491-512): known values on open faces, 0 else.
-// 990 us at 384^3 with a lane per cell, 654 in tiles, 39.7 against 52 at
-// 160 x 117 x 143; 24 bytes a cell at most, 2.1 TB/s: what is left is the sums.
+// 990 us at 384^3 with a lane per cell, 654 in tiles, 52 -> 39.7 at
+// 160 x 117 x 143, and in tiles at every size, as most tiles need no samples: 32^3
+// 22 -> 11 us, 64^3 21 -> 12, 128^3 46 -> 29; 24 bytes a cell at most, 2.1 TB/s: what is left is the sums.
 __global__ __launch_bounds__(kThreads) void k_ex_finish(ExGeo g, ExSrc src, int have_src, ExState r,
                                                        const uint8_t* __restrict__ cls, ExCounters* cnt,
                                                        float* __restrict__ uo, float* __restrict__ vo,

@@ -470,9 +470,8 @@ __device__ __forceinline__ void band_segment(const TallGeo& g, const int* __rest
 // neighbours' tall samples only where a lane's rows reach below their base.  Of
 // the seven segments of a 32-row band that reach liquid three are such and so
 // is the pair; with the surface's weights from one quotient each and every load
-// ahead of its use, at 512^2 x 34 samples a sweep takes 59 us instead of 92 (the
-// mean of a V-cycle's four), the residual 66 instead of 96, the direction 100
-// instead of 141.
+// ahead of its use, at 512^2 x 34 samples a sweep takes 74 us instead of 109, the
+// residual 71 instead of 99, the direction 108 instead of 145.
 template <class V>
 __device__ __forceinline__ void band_segment_deep(const TallGeo& g, const int* __restrict__ bases, int x, int py0,
                                                   int z, int b, const V& vec, float (&ap)[kSegRows],

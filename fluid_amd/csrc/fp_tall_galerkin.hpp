@@ -481,9 +481,8 @@ __device__ __forceinline__ void lat_prolong_node(const TallRec& G, int level, in
 // turns are dealt to the XCDs (workgroup b runs on XCD b % 8) in eight runs of
 // consecutive nodes, so that the couplings and values a node reads from its -x
 // neighbour's slab were just read on the same XCD and are in its L2 (dealt one
-// by one they came from memory: 189 MB a sweep of level 1 of 512^2 columns,
-// whose couplings and vectors are 128 MB).  A sweep there 41 -> 37 us, the
-// levels' mean 12.0 -> 10.3.
+// by one they came from memory: 184 MB read a sweep of level 1 of 512^2 columns,
+// 91 in runs).  A sweep there 34.6 -> 27.8 us, the levels' mean 12.0 -> 10.3.
 #define LAT_NODES(i, n)                                                                                    \
   for (unsigned turns_ = (unsigned)(((n) + FP_BLOCK - 1) / FP_BLOCK), xcds_ = (nblk & 7) == 0 ? 8u : 1u,   \
                 run_ = (turns_ + xcds_ - 1) / xcds_, first_ = (unsigned)blk % xcds_ * run_,                \

@@ -1221,7 +1221,7 @@ static size_t bottom_lds_grant() {
 // evaluates six weights and decodes its cell with 64-bit divisions: 428 us at
 // 384^3, whose 12 B a cell take 145.  A wave whose cells and their neighbours
 // are all air, or all liquid, knows its weights, and cell numbers below 2^32
-// are divided as such: 236 us.  (The same divisions in k_rhs, which memory
+// are divided as such: 241 us.  (The same divisions in k_rhs, which memory
 // bounds, took it from 309 to 358 us.)
 template <typename T>
 __global__ void k_build_weights(const Part* parts, int np, int level) {

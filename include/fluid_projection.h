@@ -349,8 +349,9 @@ int fp_tall_remesh(fp_grid* grid, const fp_tall_remesh_args* args, int64_t* chan
  * faces the hierarchy leaves unknown (packTransportShell, :491-512).  FP32.
  * Outputs may alias the inputs.  The first call on a grid allocates the
  * extrapolation state (about 62 bytes per cell) and the first one in host
- * memory its staging (12 more); FP_ERR_BUDGET beyond the context's budget.  Device arrays must be complete when the call is made;
- * it returns when the outputs are written. */
+ * memory its staging (12 more); FP_ERR_BUDGET beyond the context's budget.
+ * Device arrays must be complete when the call is made; it returns when the
+ * outputs are written. */
 typedef struct {
   int32_t memory;       /* FP_MEMORY_HOST or FP_MEMORY_DEVICE for the arrays below */
   int32_t open_top;     /* 1: the top (+y) faces are open to the atmosphere */
